@@ -676,6 +676,46 @@ def test_quantile_selection_value_buckets_bit_exact(gpu, B):
     assert np.array_equal(bits(got[cols]), bits(tq))
 
 
+@pytest.mark.parametrize("n,F,pad,B", [(131_072, 64, 0, 32), (131_073, 65, 3, 127),
+                                       (196_561, 1, 0, 2), (655_201, 13, 1, 10)])
+def test_two_read_quantile_edges_bit_exact(gpu, n, F, pad, B):
+    """Long columns (two reads of the matrix): row-block, 64-feature and row
+    stride remainders; smooth, lognormal, outliers, infinities, whole numbers
+    of both zero signs, mostly zeros, values crowded into one bucket, NaN and
+    constant columns, equal to the oracle bit for bit."""
+    print_case("two-read quantile edges", n, F, pad, B)
+    rng = np.random.default_rng(n)
+    X = np.full((n, F + pad), 7.0, F32)  # (the padding columns belong to no feature)
+    kinds = [
+        lambda: rng.standard_normal(n),
+        lambda: np.round(rng.standard_normal(n)),             # ties, -0.0 and +0.0
+        lambda: np.exp(2 * rng.standard_normal(n)),
+        lambda: rng.integers(0, 3000, n) // 7 * 0.5,
+        lambda: np.where(rng.random(n) < 0.97, 0.0, rng.standard_normal(n)),
+        lambda: np.where(rng.random(n) < 0.5, -0.0, rng.integers(0, 2, n)),
+        lambda: rng.standard_normal(n) * 1e-42,               # subnormal
+        lambda: np.where(np.arange(n) % 1000 == 3, np.inf, rng.standard_normal(n)),
+        lambda: np.where(np.arange(n) % 50 == 3, -np.inf, rng.standard_normal(n)),
+        lambda: np.where(rng.random(n) < 0.4, rng.random(n) * 1e-6, rng.random(n) * 1e6),
+        lambda: np.where(rng.random(n) < 0.3, 1.25, 1.25 + rng.integers(0, 4, n) * 1e-6),
+        lambda: np.where(np.arange(n) == n - 1, np.nan, rng.standard_normal(n)),
+        lambda: np.full(n, -0.0),
+    ]
+    for f in range(F):
+        X[:, f] = kinds[f % len(kinds)]()
+    Xd = torch.from_numpy(X).to(dev)
+    q = torch.from_numpy(ops.quantile_levels(B)).to(dev)
+    edges = torch.empty((F, B - 1), device=dev)
+    _lib.check(_lib.load().wgbm_quantile_edges_matrix(
+        Xd.data_ptr(), n, F, F + pad, q.data_ptr(), B - 1, edges.data_ptr(),
+        _lib.current_stream_ptr(dev)), "quantile_edges_matrix")
+    # (the radix sort orders -0.0 before +0.0, as the selection does)
+    ref = clib.quantile_edges_matrix(np.ascontiguousarray(X[:, :F]), B)
+    bad = [f for f in range(F)
+           if not np.array_equal(bits(edges[f].cpu().numpy()), bits(ref[f]))]
+    assert not bad, bad
+
+
 @pytest.mark.parametrize("B", [5, 32, 127])
 def test_staged_quantile_edges_bit_exact(gpu, B):
     """Edges taken from columns staged block by block during the upload

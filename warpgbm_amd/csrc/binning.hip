@@ -17,6 +17,7 @@
 // a NaN (NaNs sort last).
 #include "common.hpp"
 #include "kernels.hpp"
+#include "quantile_radix.hpp"
 
 namespace wgbm {
 
@@ -358,20 +359,6 @@ __global__ void quantile_edges_kernel(const float* __restrict__ sorted, int64_t 
 // prefix.  The selected keys are decoded and interpolated exactly as in
 // quantile_edges_kernel.
 // ---------------------------------------------------------------------------
-__device__ inline uint32_t float_to_key(float x) {
-  uint32_t u = __float_as_uint(x);
-  if (x != x) return 0xffffffffu;
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-// the key of a value's bits, the value not a NaN
-__device__ inline uint32_t bits_to_key(uint32_t u) {
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ inline float key_to_float(uint32_t k) {
-  const uint32_t u = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
-  return __uint_as_float(u);
-}
-
 // X [n, F] float32 (row stride xs) -> vals [F][ks] (the values' bits; ks >=
 // n, a multiple of 4, so every column starts on 16 bytes): a workgroup moves
 // 64 features x kTransRows rows in 64 x 64 tiles through LDS, and keeps the
@@ -487,8 +474,6 @@ template __global__ void transpose_values_kernel<false>(const float*, int64_t, i
                                                       int64_t, uint32_t*, uint32_t*, uint32_t*);
 
 constexpr int kSelThreads = 512;
-constexpr int kSelMaxTargets = 256;   // 2 * 126 ranks at most (num_bins <= 127)
-constexpr int kSelGroup = 32;         // distinct prefixes histogrammed per scan
 constexpr int kSelBuckets = 4096;     // value buckets of the first pass
 
 // One workgroup per feature (512 threads, ~37 KB of LDS: four per CU, so a
@@ -759,113 +744,7 @@ __global__ __launch_bounds__(kSelThreads) void quantile_select_kernel(
           if (i0 + u * kSelThreads < ns) fn(src_vals ? bits_to_key(k[u]) : k[u]);
       }
     };
-    // a 256-bin row of counts -> inclusive prefix, in place (one wave, 4 bins
-    // a lane)
-    auto row_prefix = [&](uint32_t* row) {
-      const int ln = tid & 63;
-      uint32_t v[4];
-      uint32_t t = 0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        t += row[4 * ln + j];
-        v[j] = t;
-      }
-      const uint32_t base = (uint32_t)(wgbm_wave_incl_scan_i64((int64_t)t) - t);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) row[4 * ln + j] = base + v[j];
-    };
-    // first bin whose inclusive prefix exceeds r (bins 0..255; 255 when none
-    // below does), and r made relative to that bin
-    auto pick_bin = [&](const uint32_t* P, int64_t& r) {
-      int a = 0, b = 255;
-      while (a < b) {
-        const int mid = (a + b) >> 1;
-        if ((int64_t)P[mid] > r) b = mid; else a = mid + 1;
-      }
-      if (a > 0) r -= P[a - 1];
-      return a;
-    };
-    for (int i = tid; i < nwaves * 256; i += kSelThreads) (&hist[0][0])[i] = 0;
-    __syncthreads();
-    {
-      const int w = tid >> 6;
-      for_src([&](uint32_t k) { atomicAdd(&hist[w][k >> 24], 1u); });
-    }
-    __syncthreads();
-    for (int b = tid; b < 256; b += kSelThreads) {
-      uint32_t sum = 0;
-      for (int w = 0; w < nwaves; ++w) sum += hist[w][b];
-      hist[nwaves][b] = sum;
-    }
-    __syncthreads();
-    if (tid < 64) row_prefix(hist[nwaves]);
-    __syncthreads();
-    for (int t = tid; t < nt; t += kSelThreads) {
-      int64_t r = trank[t];
-      const int b = pick_bin(hist[nwaves], r);
-      tprefix[t] = (uint32_t)b;
-      trank[t] = r;
-    }
-    __syncthreads();
-    // index of prefix pre in the sorted dist[lo..hi] (or where it would be)
-    auto find = [&](uint32_t pre, int a, int b) {
-      while (a < b) {
-        const int mid = (a + b) >> 1;
-        if (dist[mid] < pre) a = mid + 1; else b = mid;
-      }
-      return a;
-    };
-    // passes 2..4: next byte of the keys that share a target's prefix
-    for (int pass = 1; pass < 4; ++pass) {
-      const int sh = 32 - 8 * pass;  // prefix = key >> sh
-      // sorted distinct prefixes, in parallel (a serial sort on one thread
-      // waits on every LDS access behind the other waves' atomics): thread
-      // t marks whether it holds the first occurrence of its value, then a
-      // first occurrence stores its value at the count of distinct values
-      // below it
-      if (tid == 0) s_nd = 0;
-      if (tid < nt) {
-        const uint32_t v = tprefix[tid];
-        bool first = true;
-        for (int u = 0; u < tid; ++u) first = first && tprefix[u] != v;
-        tfirst[tid] = first ? 1u : 0u;
-      }
-      __syncthreads();
-      if (tid < nt && tfirst[tid]) {
-        const uint32_t v = tprefix[tid];
-        int below = 0;
-        for (int u = 0; u < nt; ++u) below += (tfirst[u] && tprefix[u] < v) ? 1 : 0;
-        dist[below] = v;
-        atomicAdd(&s_nd, 1);
-      }
-      __syncthreads();
-      const int nd = s_nd;
-      for (int g0 = 0; g0 < nd; g0 += kSelGroup) {
-        const int gn = nd - g0 < kSelGroup ? nd - g0 : kSelGroup;
-        for (int i = tid; i < gn * 256; i += kSelThreads) (&hist[0][0])[i] = 0;
-        __syncthreads();
-        const uint32_t lo_p = dist[g0], hi_p = dist[g0 + gn - 1];
-        for_src([&](uint32_t k) {
-          const uint32_t pre = k >> sh;
-          if (pre < lo_p || pre > hi_p) return;
-          const int g = find(pre, g0, g0 + gn - 1);
-          if (dist[g] == pre) atomicAdd(&hist[g - g0][(k >> (sh - 8)) & 255u], 1u);
-        });
-        __syncthreads();
-        for (int g = tid >> 6; g < gn; g += nwaves) row_prefix(hist[g]);
-        __syncthreads();
-        for (int t = tid; t < nt; t += kSelThreads) {
-          const uint32_t pre = tprefix[t];
-          if (pre < dist[g0] || pre > dist[g0 + gn - 1]) continue;
-          const int g = find(pre, g0, g0 + gn - 1);
-          int64_t r = trank[t];
-          const int b = pick_bin(hist[g - g0], r);
-          tprefix[t] = (pre << 8) | (uint32_t)b;
-          trank[t] = r;
-        }
-        __syncthreads();
-      }
-    }
+    radix_select<kSelThreads>(for_src, nt, tprefix, trank, hist, dist, tfirst, &s_nd);
   }  // !constant
   __syncthreads();
   // interpolate (torch.quantile, linear): see quantile_edges_kernel

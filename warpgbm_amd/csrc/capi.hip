@@ -644,6 +644,12 @@ int wgbm_quantile_edges_matrix(const float* X, int64_t n, int32_t n_feats, int64
   uint32_t *kmin = kmm, *kmax = kmm + chunk;
   for (int64_t f0 = 0; f0 < n_feats; f0 += chunk) {
     const int32_t fc = (int32_t)std::min<int64_t>(chunk, n_feats - f0);
+    if (n >= kQuantileTwoReadRows) {
+      const int r = launch_quantile_two_reads(X + f0, n, fc, x_stride, q, nq, edges + f0 * nq,
+                                              keys, ks, st);
+      if (r) return r;
+      continue;
+    }
     if (fill_u32(kmin, fc, 0xffffffffu, st) || fill_u32(kmax, fc, 0u, st)) return WGBM_EINVAL;
     int r = launch_stage_rows(X + f0, n, fc, x_stride, keys, ks, kmin, kmax, st);
     if (r) return r;

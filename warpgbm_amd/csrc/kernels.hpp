@@ -49,6 +49,18 @@ constexpr int kAuxStream = 3;
 constexpr int kBinTileRows = 256, kBinTileFeats = 64;
 // rows per workgroup of the key transpose of the quantile selection
 constexpr int kTransRows = 1024;
+// quantile edges in two reads (quantile.hip): value buckets, sampled values
+// per column, threads per workgroup, most rows per row block (16-bit counts)
+constexpr int kQBuckets = 1024, kQSample = 1024, kQThreads = 1024, kQMaxRows = 65520;
+// columns from this length on take the two reads, shorter ones the transposed
+// copy, whose three launches cost less than the five here.  Times in us, copy
+// / two reads, at 32 bins: 30k x 50 smooth 125 / 155, with long tails and ties
+// 219 / 161; 100k x 100 155 / 186, 483 / 219; 200k x 100 199 / 229, 855 / 304;
+// 1M x 100 757 / 440, 4019 / 614.
+constexpr int64_t kQuantileTwoReadRows = 1 << 17;
+int launch_quantile_two_reads(const float* X, int64_t n, int32_t F, int64_t xs, const float* q,
+                              int32_t nq, float* edges, uint32_t* buf, int64_t ks,
+                              hipStream_t st);
 // histogram workgroups per launch the tile sizes aim for: 2 per CU, in the
 // engine and for a single call (measured on C2: the tile kernel takes 191 us
 // against 194 us with one workgroup per CU; the finalize reads twice the
