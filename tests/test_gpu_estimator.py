@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import gbm, ops
+from oracle import clib, gbm, ops
 from tests.conftest import c1_data, print_case
 from warpgbm_amd import WarpGBM
 
@@ -252,6 +252,41 @@ def test_era_des_bins_and_blocks_bit_exact(gpu, E, B):
     assert sum(str(t).count("'feature'") for t in m.forest) > 0
     assert np.array_equal(bits(m.per_era_feature_importance_), bits(ref.imp))
     assert np.array_equal(bits(m.predict(X)), bits(ref.predict_codes(X)))
+
+
+@pytest.mark.parametrize("B,N,F,classes,chunked", [
+    (2, 40_000, 40, 0, False), (7, 27_000, 70, 0, False), (16, 9_001, 130, 0, False),
+    (17, 9_001, 65, 3, False), (32, 12_345, 260, 0, True), (64, 9_001, 129, 0, False),
+    (65, 9_001, 66, 0, False), (127, 12_345, 64, 0, False)])
+def test_era_des_tiled_levels_bit_exact(gpu, B, N, F, classes, chunked):
+    """Few large eras: the shallow levels histogram (node, era) segments over
+    row tiles and scan them from the tiles, the deeper ones take the per-segment
+    kernels; every instance of the scan, uneven eras (a dead and an empty-node
+    one among them), class trees, codes outside the bins, level chunks."""
+    print_case("estimator", "DES tiled levels", B, N, F, classes, chunked)
+    rng = np.random.default_rng(B)
+    sizes = np.array([N - N // 3 - 15, N // 3, 15])
+    era = np.repeat(np.arange(3), sizes)
+    X = rng.integers(0, B, (N, F)).astype(np.int8)
+    X[rng.random((N, F)) < 0.01] = -1
+    score = (X[:, 0] - B / 2) / B + np.where(era == 1, -0.5, 1.0) * (X[:, 1] - B / 2) / B
+    score = score + 0.2 * rng.standard_normal(N)
+    kw = dict(num_bins=B, max_depth=4, n_estimators=2, learning_rate=0.4)
+    if classes:
+        kw["objective"] = "multiclass"
+        y = np.digitize(score, np.quantile(score, [1 / 3, 2 / 3]))
+    else:
+        y = score.astype(F32)
+    m = WarpGBM(colsample_bytree=0.8, random_state=3, **kw)
+    if chunked:
+        m._engine_level_bytes = 600_000  # a few nodes per chunk
+    m.fit(X, y, era_id=era)
+    ref = gbm.Forest(**kw).fit_codes(X, y, era_id=era, feat_sets=m.feature_subsets_,
+                                     hist=clib.hist_exact_q, scan=clib.split_scan_q)
+    for i, (a, b) in enumerate(zip(m.forest, ref.forest)):
+        assert a == b, f"tree {i} differs"
+    assert sum(str(t).count("'feature'") for t in m.forest) > 10
+    assert np.array_equal(bits(m.per_era_feature_importance_), bits(ref.imp))
 
 
 def test_era_des_many_eras_blocks_bit_exact(gpu):

@@ -352,6 +352,20 @@ int launch_des_era(int V, int B, int32_t n_keys, hipStream_t st, const int8_t* c
 // the pair codes: below it the int8 kernel's smaller LDS tables keep more
 // segments (and so more row loads) in flight per CU
 constexpr int kDesPairMinRows = 96;
+// Levels of the direct era path whose (node, era) segments average at least
+// this many rows are histogrammed over row tiles and scanned from the tiles
+// (des_scan_tiles_kernel): a workgroup per segment and feature chunk leaves
+// most CUs without work there, and walks its rows one after the other.  Us per
+// round without tiles / from 2048 / from 1024 / from 256 rows: 123457 x 307, 7 eras, 63
+// bins, depth 6: 1166 / 714 / 717 / 727; 300k x 300, 20 eras, 32 bins: 1082 /
+// 619 / 615 / 607; 200k x 500, 20 eras, 10 bins: 834 / 550 / 540 / 579; 300k x
+// 300, 101 eras, 10 bins: 649 / 635 / 643 / 677; 50k x 100, 3 eras: 718 / 279 /
+// 281 / 277.
+constexpr int64_t kEraTileRows = 1024;
+// with pair codes, whose kernel adds half as many words per row, from longer
+// segments on (without / from 8192 / from 2048): 500k x 500, 20 eras, 5 bins 839 /
+// 699 / 716; 300k x 300, 101 eras 464 / 479 / 496
+constexpr int64_t kEraTileRowsPair = 8192;
 int launch_pack_pairs(hipStream_t st, const int8_t* codes, int64_t stride, int32_t F, int64_t n,
                       int32_t B, uint8_t* out, int64_t pstride);
 // row stride of the pair codes: one byte per feature pair, whole 8-byte

@@ -79,6 +79,7 @@ struct Engine {
   int64_t pstride = 0;
   bool pcodes_ready = false;
   int des_codes = 1;
+  bool era_tiles = true;  // levels of few large segments over tiles (era_level_tiles)
   // one-era levels: 1 = level_scan_e1_kernel (a thread per node), 0 = the
   // wave-per-node kernels
   int lscan_e1 = 1;
@@ -471,12 +472,49 @@ static int level_plan(Engine* e, int d, LevelPlan* lp) {
   return ensure_tiles(e, lp->max_tiles);
 }
 
+// direct era levels of few large segments (era_level_tiles): the tiles of nc
+// (tree, node)s, the level split into n_chunk such runs
+static void era_tile_sizes(const Engine* e, int64_t nc, int n_chunk, LevelPlan* lp) {
+  const int64_t TN = (int64_t)e->c.n_trees * e->c.n_rows;
+  lp->n_list = (int32_t)(nc * e->c.num_eras);
+  lp->rows_bound = TN;
+  lp->R = pick_tile_rows(e, std::max<int64_t>(1, TN / std::max(n_chunk, 1)));
+  lp->max_tiles = TN / lp->R + lp->n_list + 1;
+}
+
+static int era_tile_plan(Engine* e, int64_t nc, int n_chunk, LevelPlan* lp) {
+  era_tile_sizes(e, nc, n_chunk, lp);
+  return ensure_tiles(e, lp->max_tiles);
+}
+
+// whether depth d of the direct era path takes tiles: by the mean rows of a
+// (node, era) segment (see kEraTileRows)
+static bool era_level_tiles(const Engine* e, int d) {
+  if (!e->era_tiles) return false;
+  const int64_t rows = e->pcodes && e->des_codes == 1 ? kEraTileRowsPair : kEraTileRows;
+  return e->c.n_rows >= rows * (int64_t(1) << d) * e->c.num_eras;
+}
+
 // the tile buffers of every whole level a round histograms, sized once before
 // the first round's launches: growing them level by level would synchronise
 // the device (a buffer in use is freed only after a sync) at each depth
 static int presize_levels(Engine* e) {
-  if (e->des_direct) return 0;
   int64_t mt = 0;
+  if (e->des_direct) {
+    for (int d = 0; d < e->c.max_depth && era_level_tiles(e, d); ++d) {
+      const int64_t n_tn = (int64_t)e->c.n_trees << d, nc = std::min(e->nc_max, n_tn);
+      LevelPlan lp;
+      era_tile_sizes(e, nc, (int)((n_tn + nc - 1) / nc), &lp);
+      mt = std::max(mt, lp.max_tiles);
+    }
+    const int r = mt > 0 ? ensure_tiles(e, mt) : 0;
+    if (r != WGBM_ENOMEM) return r;
+    // no room for the tiles' partials: every level takes the per-segment
+    // kernels, which need none
+    (void)hipGetLastError();
+    e->era_tiles = false;
+    return 0;
+  }
   for (int d = 0; d < e->c.max_depth; ++d) {
     // levels take the subtraction path while every level so far fits whole
     if (((int64_t)e->c.n_trees << d) > e->nc_max) break;
@@ -496,6 +534,30 @@ static int chunk_plan(Engine* e, int64_t n_list, int n_chunk, LevelPlan* lp) {
   lp->R = pick_tile_rows(e, std::max<int64_t>(1, TN / std::max(n_chunk, 1)));
   lp->max_tiles = TN / lp->R + n_list + 1;
   return ensure_tiles(e, lp->max_tiles);
+}
+
+// the histogram launch of the current level's tiles (the caller adds them):
+// residuals in position order, quantised with the shift of each tile's key
+// (the (tree, node) with one era, the (tree, node, era) segment with several)
+static HistLaunch level_hist(const Engine* e, int cur, int64_t k0) {
+  HistLaunch a;
+  a.codes = e->c.codes_rm;
+  a.n_rows = e->c.n_rows;
+  a.stride = e->c.stride;
+  a.n_feats = e->c.n_feats;
+  a.resid = e->rpos[cur];
+  a.resid_by_pos = 1;
+  a.resid_tree_stride = 0;
+  a.shifts = e->node_shift[cur] + k0;
+  a.order = e->order[cur];
+  a.keys_per_tree = 1;
+  a.num_bins = e->c.num_bins;
+  a.part = e->part;
+  a.V = e->V;
+  a.n_chunks = e->n_chunks;
+  a.native = 1;  // the engine's codes come from the library's binner / pre-binned copy
+  a.timer_tag = "engine_hist_tiles";
+  return a;
 }
 
 static inline unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -619,7 +681,8 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
       // ---- E > 1, direct: per-era gains of every (node, era) segment
       const int64_t ncand = (int64_t)n_sel * (B - 1);
       // pair codes for levels of large segments (mean rows per (node, era))
-      const bool use_pairs = e->pcodes && e->des_codes == 1 &&
+      const bool use_tiles = era_level_tiles(e, d);
+      const bool use_pairs = !use_tiles && e->pcodes && e->des_codes == 1 &&
                              N >= (int64_t)kDesPairMinRows * nodes * E;
       if (use_pairs && !e->pcodes_ready) {
         int r = launch_pack_pairs(st, c.codes_rm, c.stride, F, N, B, e->pcodes, e->pstride);
@@ -638,10 +701,33 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
         snprintf(tag, sizeof tag, "des_rows_L%d", d);
         void* tm = timer_mode() == 1 ? timer_begin(tag) : nullptr;
         if (tm) WGBM_CHECK(hipEventRecord(timer_start_event(tm), st));
-        int r = launch_des_era(e->V, B, nc * E, st, c.codes_rm, c.stride, F, e->rpos[cur],
-                               e->node_shift[cur] + k0, e->order[cur], e->seg[cur] + k0, E, nodes,
-                               e->present[cur] + c0, e->local_of, n_sel, mcw, eps, e->sgain,
-                               e->sdir, use_pairs ? e->pcodes : nullptr, N, e->pstride);
+        int r = 0;
+        if (use_tiles) {
+          // few large segments: split over tiles, then scanned from the tiles
+          LevelPlan lp;
+          r = era_tile_plan(e, nc, (n_tn + nc - 1) / nc, &lp);
+          if (r) return r;
+          hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
+                             (int64_t)0, lp.n_list, (const int32_t*)nullptr, (int32_t)lp.R, 0,
+                             (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
+                             e->present[cur] + c0, E, mcw);
+          WGBM_LAUNCH_CHECK();
+          HistLaunch a = level_hist(e, cur, k0);
+          a.tiles = e->htiles;
+          a.n_tiles = e->hn;
+          a.max_tiles = (int32_t)lp.max_tiles;
+          r = launch_hist_tiles(a, st);
+          if (r) return r;
+          r = launch_des_scan_tiles(e->part, e->hkts, e->hn, lp.n_list, e->n_chunks, e->V, B, F, E,
+                                    e->seg[cur] + k0, e->present[cur] + c0,
+                                    e->node_shift[cur] + k0, e->local_of, n_sel, mcw, eps,
+                                    e->sgain, e->sdir, st);
+        } else {
+          r = launch_des_era(e->V, B, nc * E, st, c.codes_rm, c.stride, F, e->rpos[cur],
+                             e->node_shift[cur] + k0, e->order[cur], e->seg[cur] + k0, E, nodes,
+                             e->present[cur] + c0, e->local_of, n_sel, mcw, eps, e->sgain,
+                             e->sdir, use_pairs ? e->pcodes : nullptr, N, e->pstride);
+        }
         if (r) return r;
         if (tm) {
           WGBM_CHECK(hipEventRecord(timer_stop_event(tm), st));
@@ -723,7 +809,8 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
             }
             hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur],
                                (int64_t)0, n_list, list, (int32_t)R, 0, (int32_t)max_tiles,
-                               e->root_tiles, e->root_kts, e->root_hn);
+                               e->root_tiles, e->root_kts, e->root_hn, (const int32_t*)nullptr, 1,
+                               0.0f);
             WGBM_LAUNCH_CHECK();
             e->root_tiles_ready = true;
           }
@@ -733,31 +820,13 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
         } else if (!(subtract && planned)) {
           hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
                              (int64_t)0, n_list, list, (int32_t)R, 0, (int32_t)max_tiles,
-                             e->htiles, e->hkts, e->hn);
+                             e->htiles, e->hkts, e->hn, (const int32_t*)nullptr, 1, 0.0f);
           WGBM_LAUNCH_CHECK();
         }
-        HistLaunch a;
-        a.codes = c.codes_rm;
-        a.n_rows = N;
-        a.stride = c.stride;
-        a.n_feats = F;
-        a.resid = e->rpos[cur];  // residuals in position order (global positions)
-        a.resid_by_pos = 1;
-        a.resid_tree_stride = 0;
-        // quantised with the histogram shift of each tile's key (the (tree,
-        // node) with one era, the (tree, node, era) segment with several)
-        a.shifts = e->node_shift[cur] + k0;
-        a.order = e->order[cur];
+        HistLaunch a = level_hist(e, cur, k0);
         a.tiles = tl_d;
         a.n_tiles = hn_d;
-        a.keys_per_tree = 1;
-        a.num_bins = B;
-        a.part = e->part;
-        a.V = e->V;
-        a.n_chunks = e->n_chunks;
         a.max_tiles = (int32_t)max_tiles;
-        a.native = 1;  // the engine's codes come from the library's binner / pre-binned copy
-        a.timer_tag = "engine_hist_tiles";
         r = launch_hist_tiles(a, st);
         if (r) return r;
         const int64_t pairs = (subtract && d > 0) ? n_list / 2 : n_list;

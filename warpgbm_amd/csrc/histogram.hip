@@ -29,6 +29,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
+#include "split_scan.hpp"
 
 namespace wgbm {
 
@@ -746,6 +747,109 @@ __global__ __launch_bounds__(PT) void hist_finalize_plane_level_kernel(
 }
 
 // --------------------------------------------------------------------------
+// Split scan of few, large (node, era) segments from their tile partials (the
+// staged gains and directions of des_era_kernel, which histograms a segment
+// in one workgroup and leaves the GPU idle when there are few): one workgroup
+// per (segment, plane) sums the segment's tiles as the plane finalize does,
+// one thread per feature walks its bins in order (the sequential float32
+// sums), and all threads evaluate the candidates from those prefixes.
+// Bound by the partials' reads and the staged stores; where it is taken, and
+// what it measured, see kEraTileRows.
+// --------------------------------------------------------------------------
+template <int MB, int PT, int PG>
+__global__ __launch_bounds__(PT) void des_scan_tiles_kernel(
+    const unsigned long long* __restrict__ part, const int32_t* __restrict__ key_tile_start,
+    const int32_t* __restrict__ n_tiles, int32_t n_keys, int32_t n_chunks, int32_t V,
+    int32_t num_bins, int32_t n_feats, int32_t E, const int64_t* __restrict__ seg,
+    const int32_t* __restrict__ present, const int32_t* __restrict__ key_shift,
+    const int32_t* __restrict__ local_of, int32_t n_sel, float mcw, float eps,
+    float* __restrict__ gain, int8_t* __restrict__ dir) {
+  __shared__ unsigned long long sq[MB * kPlaneRow];
+  __shared__ unsigned int sc[MB * kPlaneRow];
+  __shared__ float tot_g[kHistSlots], tot_h[kHistSlots];
+  __shared__ int32_t loc[kHistSlots];
+  const int P = n_chunks * V;
+  const int key = (int)blockIdx.x / P;
+  const int plane = (int)blockIdx.x - key * P;
+  if (key >= n_keys) return;  // uniform per workgroup
+  const int tn = key / E, era = key - (key / E) * E;
+  if (!present[tn] || des_segment_dead(seg[key + 1] - seg[key], mcw)) return;  // uniform
+  const int chunk = plane / V, j = plane - (plane / V) * V;
+  const int tid = threadIdx.x;
+  if (tid < kHistSlots) {
+    const int f = chunk * kHistSlots * V + tid * V + j;
+    loc[tid] = f < n_feats ? local_of[f] : -1;
+  }
+  const int64_t tile_words = (int64_t)n_chunks * kHistSlots * V * num_bins;
+  const int t0 = key_tile_start[key], nt = *n_tiles;
+  const int t1 = key_tile_start[key + 1] < nt ? key_tile_start[key + 1] : nt;
+  plane_sum<MB, PT, PG>(part, tile_words, plane * num_bins * kHistSlots, num_bins, t0, t1, sq,
+                        sc);
+  const int s = key_shift[key];
+  // each bin's float sum and count over its words: the low half of the sum's
+  // word and the count's word
+  float* gf = reinterpret_cast<float*>(sq);  // word li at 2 * li
+  float* hf = reinterpret_cast<float*>(sc);
+  for (int o = tid; o < num_bins * kHistSlots; o += PT) {
+    const int li = (o / kHistSlots) * kPlaneRow + o % kHistSlots;
+    const float g = wgbm_dequantise((int64_t)sq[li], s);
+    const float h = (float)(int32_t)sc[li];
+    gf[2 * li] = g;
+    hf[li] = h;
+  }
+  __syncthreads();
+  if (tid < kHistSlots && loc[tid] >= 0) {
+    // totals, then prefixes in place, as scan_bins adds them
+    float Gt = 0.0f, Ht = 0.0f;
+    for (int b = 0; b < num_bins; ++b) {
+      Gt = Gt + gf[2 * (b * kPlaneRow + tid)];
+      Ht = Ht + hf[b * kPlaneRow + tid];
+      gf[2 * (b * kPlaneRow + tid)] = Gt;
+      hf[b * kPlaneRow + tid] = Ht;
+    }
+    tot_g[tid] = Gt;
+    tot_h[tid] = Ht;
+  }
+  __syncthreads();
+  const int nb = num_bins - 1;
+  const int W = (E + kDesEraBlock - 1) / kDesEraBlock;
+  const int64_t c64 = ((int64_t)n_sel * nb + 63) / 64;
+  for (int o = tid; o < nb * kHistSlots; o += PT) {
+    const int lane = o / nb, b = o - lane * nb;
+    const int l = loc[lane];
+    if (l < 0) continue;
+    float g, d;
+    split_candidate(gf[2 * (b * kPlaneRow + lane)], hf[b * kPlaneRow + lane], tot_g[lane],
+                    tot_h[lane], mcw, eps, g, d);
+    const int64_t slot = des_stage_slot(tn, era, W, c64, (int64_t)l * nb + b);
+    gain[slot] = g;
+    dir[slot] = (int8_t)d;
+  }
+}
+
+int launch_des_scan_tiles(const unsigned long long* part, const int32_t* key_tile_start,
+                          const int32_t* n_tiles, int32_t n_keys, int32_t n_chunks, int32_t V,
+                          int32_t num_bins, int32_t n_feats, int32_t E, const int64_t* seg,
+                          const int32_t* present, const int32_t* key_shift,
+                          const int32_t* local_of, int32_t n_sel, float mcw, float eps,
+                          float* gain, int8_t* dir, hipStream_t st) {
+  const int64_t wg = (int64_t)n_keys * n_chunks * V;
+  WGBM_REQUIRE(wg < ((int64_t)1 << 31), "era scan: too many segments");
+  WGBM_REQUIRE(num_bins <= 128, "era scan: at most 128 bins");
+#define WGBM_L(MB, PT, PG)                                                                     \
+  hipLaunchKernelGGL((des_scan_tiles_kernel<MB, PT, PG>), dim3((unsigned)wg), dim3(PT), 0, st, \
+                     part, key_tile_start, n_tiles, n_keys, n_chunks, V, num_bins, n_feats, E, \
+                     seg, present, key_shift, local_of, n_sel, mcw, eps, gain, dir)
+  if (num_bins <= 16) WGBM_L(16, 256, 1);
+  else if (num_bins <= 32) WGBM_L(32, 512, 2);
+  else if (num_bins <= 64) WGBM_L(64, 1024, 4);
+  else WGBM_L(128, 1024, 1);
+#undef WGBM_L
+  WGBM_LAUNCH_CHECK();
+  return 0;
+}
+
+// --------------------------------------------------------------------------
 // finalize for the level-wise engine: exact int64 sums into the level arrays,
 // plus the sibling histogram as (parent - computed child), also exact.
 //   computed key k = (tree, node, era) with node = 2*parent + side
@@ -979,9 +1083,10 @@ __global__ __launch_bounds__(1024) void plan_tiles_kernel(
     const int64_t* __restrict__ seg, int64_t total_rows, int32_t n_keys,
     const int32_t* __restrict__ key_list, int32_t tile_rows, int32_t nearest,
     int32_t max_tiles, Tile* __restrict__ tiles, int32_t* __restrict__ key_tile_start,
-    int32_t* __restrict__ n_tiles) {
+    int32_t* __restrict__ n_tiles, const int32_t* __restrict__ present, int32_t num_eras,
+    float mcw) {
   plan_tiles_body(seg, total_rows, n_keys, key_list, tile_rows, nearest, max_tiles, tiles,
-                  key_tile_start, n_tiles);
+                  key_tile_start, n_tiles, present, num_eras, mcw);
 }
 
 

@@ -186,7 +186,14 @@ __global__ void absmax_finish_kernel(const uint32_t* partial, int32_t n_part, in
 __global__ void plan_tiles_kernel(const int64_t* seg, int64_t total, int32_t n_keys,
                                   const int32_t* key_list, int32_t tile_rows, int32_t nearest,
                                   int32_t max_tiles, Tile* tiles, int32_t* key_tile_start,
-                                  int32_t* n_tiles);
+                                  int32_t* n_tiles, const int32_t* present, int32_t num_eras,
+                                  float mcw);
+int launch_des_scan_tiles(const unsigned long long* part, const int32_t* key_tile_start,
+                          const int32_t* n_tiles, int32_t n_keys, int32_t n_chunks, int32_t V,
+                          int32_t num_bins, int32_t n_feats, int32_t E, const int64_t* seg,
+                          const int32_t* present, const int32_t* key_shift,
+                          const int32_t* local_of, int32_t n_sel, float mcw, float eps,
+                          float* gain, int8_t* dir, hipStream_t st);
 __global__ void hist_prep_kernel(const float* resid, const int32_t* rows, int64_t n,
                                  uint32_t* partial, float* gathered, int32_t n_part, int32_t plan,
                                  const int64_t* seg, int32_t n_keys, int32_t tile_rows,

@@ -2,6 +2,7 @@
 #pragma once
 #include "common.hpp"
 #include "kernels.hpp"
+#include "split_scan.hpp"
 
 namespace wgbm {
 
@@ -14,13 +15,16 @@ namespace wgbm {
 // a small remainder, so the workgroups of a launch carry even work.  keys:
 // either all n_keys (list == nullptr) or the first *n_list entries of
 // key_list.  seg: int64 [n_keys+1] (nullptr => a single segment [0, total)).
+// With present (and no list), keys of an absent node (key / num_eras) and
+// dead segments (des_segment_dead) get no tiles.
 // --------------------------------------------------------------------------
 // (blockDim.x == 1024)
 __device__ inline void plan_tiles_body(
     const int64_t* __restrict__ seg, int64_t total_rows, int32_t n_keys,
     const int32_t* __restrict__ key_list, int32_t tile_rows, int32_t nearest,
     int32_t max_tiles, Tile* __restrict__ tiles, int32_t* __restrict__ key_tile_start,
-    int32_t* __restrict__ n_tiles) {
+    int32_t* __restrict__ n_tiles, const int32_t* __restrict__ present = nullptr,
+    int32_t num_eras = 1, float mcw = 0.0f) {
   __shared__ int64_t wsum[16];
   __shared__ int64_t sbuf[kScanK * 1024];
   const int nk = n_keys;  // entries of key_list (or keys 0..n_keys-1)
@@ -28,6 +32,7 @@ __device__ inline void plan_tiles_body(
     key = key_list ? key_list[i] : i;
     b0 = (key >= 0 && seg) ? seg[key] : 0;
     b1 = key < 0 ? 0 : (seg ? seg[key + 1] : total_rows);
+    if (present && (!present[key / num_eras] || des_segment_dead(b1 - b0, mcw))) key = -1;
   };
   // segment lengths are below 2^31 (positions are int32): 32-bit divisions
   auto count = [&](int64_t len64) -> int64_t {

@@ -18,6 +18,23 @@ struct ScanOut {
   float dir;
 };
 
+// Gain and direction of the cut whose left side holds (GL, HL) of a node's
+// totals (Gt, Ht); the expressions and their order are those of scan_bins.
+__device__ inline void split_candidate(float GL, float HL, float Gt, float Ht, float mcw,
+                                       float eps, float& gain, float& dir) {
+  const float GR = Gt - GL;
+  const float HR = Ht - HL;
+  gain = 0.0f;
+  dir = 0.0f;
+  if (HL >= mcw && HR >= mcw) {
+    const float tot = (Gt * Gt) / (Ht + eps);
+    gain = (GL * GL) / (HL + eps) + (GR * GR) / (HR + eps) - tot;
+    const float lv = GL / (HL + eps);
+    const float rv = GR / (HR + eps);
+    dir = lv > rv ? 1.0f : -1.0f;
+  }
+}
+
 // sequential scan of one (era, feature) histogram; calls emit(b, gain, dir)
 template <typename LoadG, typename LoadH, typename Emit>
 __device__ inline void scan_bins(int B, float mcw, float eps, LoadG g, LoadH h, Emit emit) {
