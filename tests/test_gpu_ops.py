@@ -423,6 +423,36 @@ def test_predict_heap_paths_bit_exact(gpu, case):
     assert np.array_equal(bits(out.cpu().numpy()), bits(ref))
 
 
+# rows, features, bins, classes, rounds, depth: the column-block predictor's row
+# blocks (256) and stride groups (16 columns), values through LDS (below 8
+# classes) or sums in registers (one or two classes a wave, to 32), the extension
+# of trees shallower than 4, bins up to the largest, partial chunks
+COLS_CASES = [
+    (1, 1, 2, 1, 3, 1), (255, 16, 127, 1, 40, 4), (257, 17, 32, 7, 9, 3), (700, 33, 10, 8, 30, 6),
+    (1025, 300, 32, 17, 5, 5), (513, 120, 127, 32, 4, 2), (300, 380, 63, 3, 12, 8),
+    (300, 50, 16, 33, 3, 5), (300, 505, 16, 9, 3, 6),
+]
+
+
+@pytest.mark.parametrize("case", COLS_CASES, ids=[str(c) for c in COLS_CASES])
+def test_predict_heap_column_blocks_bit_exact(gpu, case):
+    """wgbm_predict_heap against the reference-table walk at the edges of the
+    column-block predictor, codes outside [0, B) and single-leaf trees
+    included, and one case past each of its limits."""
+    N, F, B, K, R, depth = case
+    print_case("predict_heap column blocks", case)
+    rng = np.random.default_rng(N + F)
+    raw = rng.integers(-2, min(B + 3, 128), (N, F)).astype(np.int8)
+    feat, binv, leaf, tables = _random_heap(rng, R, K, depth, F, B)
+    out0 = rng.standard_normal((N, K)).astype(F32)
+    codes = D.codes_from_int8(D.upload_int8(raw, dev), False, B)[0]
+    out = t(out0)
+    D.predict_heap(codes, t(feat), t(binv), t(leaf), R, K, depth, 0.1, out)
+    cls = np.tile(np.arange(K, dtype=np.int32), R)
+    ref = clib.predict_tables(raw, tables, F32(0.1), out0, cls)
+    assert np.array_equal(bits(out.cpu().numpy()), bits(ref))
+
+
 def native_layout(raw, num_bins, stride):
     """The library's native row-major code layout (include/warpgbm_amd.h):
     codes in [0, B) as is, negative codes B, codes >= B and padding B + 1."""

@@ -407,6 +407,40 @@ static int predict_heap_impl(const int8_t* codes, int64_t n, int64_t codes_strid
   WGBM_CHECK(hipGetDevice(&dev));
   WGBM_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
   const bool resident = predict_resident_plan(codes_stride, K, H, n_rounds, &RB, &lds) != 0;
+  // The column-block predictor where two of its workgroups share a CU, or
+  // nothing else keeps the trees in LDS.  1M x 100, 32 bins, us with the row
+  // walkers / with it: 2000 trees of depth 6, 10 classes 3600 / 1910; 100 trees,
+  // one class: depth 6 239 / 169, depth 5 213 / 136, depth 3 161 / 128; 200k x
+  // 300, 3 classes, 300 trees of depth 8 430 / 243; but one workgroup a CU,
+  // 200k x 300, 100 trees of depth 5: 64 / 81.
+  int32_t DX = 0, waves = 0, cols_tc = 0;
+  bool vt = false;
+  size_t cols_lds = 0;
+  if (predict_cols_plan(codes_stride, K, max_depth, n_rounds, &DX, &waves, &cols_tc, &vt,
+                        &cols_lds) &&
+      (uintptr_t)codes % 16 == 0 && (!resident || cols_lds <= 80 * 1024)) {
+    const int64_t T = (int64_t)n_rounds * K, words = kColsUni + (int64_t(2) << DX) - (1 << kColsTop);
+    uint32_t* uni = (uint32_t*)scratch_get(S(stream), sizeof(uint32_t) * (size_t)(T * words), 13);
+    WGBM_REQUIRE(uni, "scratch allocation failed");
+    uint32_t* tab = uni + T * kColsUni;
+    hipLaunchKernelGGL(cols_tables_kernel, dim3(nblocks(T * words, 256)), dim3(256), 0, S(stream),
+                       feat, bin, leaf, T, max_depth, DX, codes_stride, learning_rate, uni, tab);
+    WGBM_LAUNCH_CHECK();
+    static bool attr_c = false;
+    if (!attr_c) {
+      WGBM_CHECK(hipFuncSetAttribute((const void*)predict_cols_kernel<true>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+      WGBM_CHECK(hipFuncSetAttribute((const void*)predict_cols_kernel<false>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+      attr_c = true;
+    }
+    hipLaunchKernelGGL((vt ? predict_cols_kernel<true> : predict_cols_kernel<false>),
+                       dim3(nblocks(n, kColsRows)), dim3(64 * waves), cols_lds, S(stream), codes,
+                       n, codes_stride, num_bins, (const uint32_t*)uni, (const uint32_t*)tab,
+                       (int32_t)T, K, DX, cols_tc, out, skip);
+    WGBM_LAUNCH_CHECK();
+    return 0;
+  }
   const bool rows = !resident && predict_rows_plan(codes_stride, K, H, n_rounds, &RB, &TC, &lds);
   uint32_t* cnode = nullptr;
   float* cleaf = nullptr;
@@ -727,7 +761,9 @@ int wgbm_softmax_rows(float* x, int64_t n, int32_t K, void* stream) {
   WGBM_REQUIRE(n >= 0 && K >= 1, "bad softmax shape");
   if (n == 0) return 0;
   WGBM_REQUIRE(x, "null pointer");
-  hipLaunchKernelGGL(softmax_rows_kernel, dim3(nblocks(n, 256)), dim3(256), 0, S(stream), x, n, K);
+  const size_t lds = K <= kSoftmaxLds ? sizeof(float) * 256 * (size_t)(K | 1) : 0;
+  hipLaunchKernelGGL(softmax_rows_kernel, dim3(nblocks(n, 256)), dim3(256), lds, S(stream), x, n,
+                     K);
   WGBM_LAUNCH_CHECK();
   return 0;
 }

@@ -413,6 +413,20 @@ __global__ void predict_heap_kernel(const int8_t* codes, int64_t n, int64_t S, i
 __global__ void complete_tables_kernel(const int32_t* feat, const int32_t* bin, const float* leaf,
                                        int64_t T, int32_t D, int64_t S, float lr,
                                        uint32_t* cnode, float* cleaf);
+// column-block predictor: top levels evaluated whole, their words per tree
+// (padded), (row, class) sums per thread, rows per workgroup
+constexpr int kSoftmaxLds = 32;  // classes of a row softmax staged in LDS (33 KB)
+constexpr int kColsTop = 4, kColsUni = 8, kColsMaxAcc = 8, kColsRows = 256;
+__global__ void cols_tables_kernel(const int32_t* feat, const int32_t* bin, const float* leaf,
+                                   int64_t T, int32_t D, int32_t DX, int64_t S, float lr,
+                                   uint32_t* uni, uint32_t* tab);
+template <bool VT>
+__global__ void predict_cols_kernel(const int8_t* codes, int64_t n, int64_t S, int32_t num_bins,
+                                    const uint32_t* uni, const uint32_t* tab, int32_t T,
+                                    int32_t K, int32_t DX, int32_t TC, float* out,
+                                    const int32_t* skip);
+int predict_cols_plan(int64_t S, int32_t K, int32_t D, int32_t n_rounds, int32_t* DX_out,
+                      int32_t* waves_out, int32_t* TC_out, bool* vt_out, size_t* lds_out);
 __global__ void predict_rows_kernel(const int8_t* codes, int64_t n, int64_t S, int32_t num_bins,
                                     const uint32_t* cnode, const float* cleaf, int32_t n_rounds,
                                     int32_t K, int32_t max_depth, int32_t RB, int32_t TC,

@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "engine.hpp"
 #include "kernels.hpp"
 
 namespace wgbm {
@@ -576,20 +577,315 @@ int predict_rows_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int32_t
   return 1;
 }
 
-// in-place row softmax over K logits: exp(x - max) / sum, sequential in k
-__global__ void softmax_rows_kernel(float* __restrict__ x, int64_t n, int32_t K) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float* r = x + i * K;
-  float m = r[0];
-  for (int k = 1; k < K; ++k) m = r[k] > m ? r[k] : m;
-  float s = 0.0f;
-  for (int k = 0; k < K; ++k) {
-    const float e = wgbm_expf(r[k] - m);
-    r[k] = e;
-    s = s + e;
+// ---------------------------------------------------------------------------
+// Column-block inference (same results as predict_rows_kernel): a workgroup
+// holds 256 rows in LDS transposed, word (f, lane) = the code bytes of rows
+// lane, lane + 64, lane + 128, lane + 192 at feature f, so a lane reads only
+// its own bank whatever features its rows are at, and one word serves four
+// rows.  A wave walks one tree for all 256 rows:
+//   * the first kColsTop levels are evaluated for every node (the node words
+//     are wave-uniform scalar loads): a code byte c goes right at bin b iff c
+//     + (127 - b) has bit 7 set, four rows in one add, and each level's bits
+//     select among the next level's (bit select) -- 15 word reads and no
+//     node reads for 4 rows x 4 levels, where walking takes 32 byte and node
+//     reads;
+//   * the levels below, and the leaf, are walked row by row: a level's node
+//     words are at most 64 consecutive words at the usual depths, so lanes at
+//     different nodes read different banks.
+// A leaf above the last level, or a tree shallower than kColsTop, continues as
+// always-left nodes (complete tables).  Each class's trees are added in tree
+// order: with VT = false wave w keeps the sums of classes w, w + waves, ... in
+// registers; with VT = true (few classes) the waves share the chunk's trees,
+// write each tree's values to LDS and one thread per (row, class) adds them.
+// The row-at-a-time walkers take 12 reads a row and tree at depth 6, 39% of the
+// LDS's cycles in conflicts of the row bytes; here it is 35 reads and 111 VALU
+// instructions for 256 rows, which bound it about equally (2000 trees of depth
+// 6 on 1M rows of 100 features: 3.60 -> 1.91 ms).
+//   LDS: columns [S + 1][64] words (the last is zero: the always-left node's
+//   column), the chunk's tables [TC][GW], values [TC][256] (VT).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kBit7 = 0x80808080u;
+
+// Per tree: kColsUni words, two top-level nodes each (column << 7 | 127 - bin;
+// an always-left node names the zero column S with addend 0), then GW =
+// 2^(D' + 1) - 2^kColsTop words, D' = max(D, kColsTop): the nodes below
+// (column << 8 | bin; always left: bin 255) by heap index (1-based), and the
+// 2^D' leaf values times lr (rounded to float32).
+__global__ void cols_tables_kernel(const int32_t* __restrict__ feat,
+                                   const int32_t* __restrict__ bin,
+                                   const float* __restrict__ leaf, int64_t T, int32_t D,
+                                   int32_t DX, int64_t S, float lr, uint32_t* __restrict__ uni,
+                                   uint32_t* __restrict__ tab) {
+  const int H = (2 << D) - 1;
+  const int GW = (2 << DX) - (1 << kColsTop);
+  const int per = kColsUni + GW;
+  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (gid >= T * per) return;
+  const int64_t t = gid / per;
+  const int j = (int)(gid - t * per);
+  const int32_t* ft = feat + t * H;
+  const bool top = j < kColsUni;
+  // node word of heap index g: column and bin (always left: the zero column S
+  // and 255)
+  auto node = [&](int g, uint32_t& f, uint32_t& b) {
+    const int d = 31 - __builtin_clz((unsigned)g);
+    bool split = d < D;
+    for (int k = 0; k <= d && split; ++k) split = ft[(g >> (d - k)) - 1] >= 0;
+    f = (uint32_t)S;
+    b = 255u;
+    if (split) {
+      f = (uint32_t)(ft[g - 1] < S ? ft[g - 1] : S - 1);
+      b = (uint32_t)bin[t * H + g - 1] & 0xffu;
+    }
+  };
+  uint32_t f = 0, b = 0;
+  if (top) {
+    uint32_t w = 0;
+    for (int h = 0; h < 2; ++h) {
+      const int gt = 2 * j + h + 1;
+      if (gt >= (1 << kColsTop)) break;  // padding
+      node(gt, f, b);
+      // code bytes are at most 128: no byte goes right of a bin above 127
+      const uint32_t x = b <= 127u ? f << 7 | (127u - b) : (uint32_t)S << 7;
+      w |= x << (16 * h);
+    }
+    uni[t * kColsUni + j] = w;
+    return;
   }
-  for (int k = 0; k < K; ++k) r[k] = r[k] / s;
+  const int g = j - kColsUni + (1 << kColsTop);
+  if (g < (1 << DX)) {
+    node(g, f, b);
+    tab[t * GW + j - kColsUni] = f << 8 | b;
+    return;
+  }
+  // leaf slot: the first node that is not a split on the path to its ancestor
+  // at depth D
+  const int h = (g >> (DX - D)) - 1;
+  int a = h;
+  for (int k = 0; k < D; ++k) {
+    const int ak = ((h + 1) >> (D - k)) - 1;
+    if (ft[ak] < 0) {
+      a = ak;
+      break;
+    }
+  }
+  tab[t * GW + j - kColsUni] = __float_as_uint(lr * leaf[t * H + a]);
+}
+
+__device__ __forceinline__ uint32_t bit_select(uint32_t m, uint32_t a, uint32_t b) {
+  return (m & a) | (~m & b);  // v_bfi_b32
+}
+
+template <bool VT>
+__global__ __launch_bounds__(1024) void predict_cols_kernel(
+    const int8_t* __restrict__ codes, int64_t n, int64_t S, int32_t num_bins,
+    const uint32_t* __restrict__ uni, const uint32_t* __restrict__ tab, int32_t T, int32_t K,
+    int32_t DX, int32_t TC, float* __restrict__ out, const int32_t* __restrict__ skip) {
+  if (skip && *skip) return;  // uniform: the caller's fallback runs instead
+  extern __shared__ uint32_t psm[];
+  const int GW = (2 << DX) - (1 << kColsTop);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nw = blockDim.x >> 6;
+  uint32_t* cols = psm;                        // [S + 1][64]
+  uint32_t* tabs = psm + (S + 1) * 64;         // [TC][GW]
+  float* vals = reinterpret_cast<float*>(tabs + TC * GW);  // [TC][256] (VT)
+  const int64_t row0 = (int64_t)blockIdx.x * kColsRows;
+  const uint32_t bb = (uint32_t)num_bins * 0x01010101u;
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  // stage: thread (lane, 16-column group) transposes 4 rows x 16 bytes
+  for (int q = wave; q < (int)(S / 16); q += nw) {
+    u4 x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t r = row0 + lane + 64 * j;
+      x[j] = *(reinterpret_cast<const u4*>(codes + (r < n ? r : n - 1) * S) + q);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint32_t y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = walk_bytes(x[j][c], bb);
+      const uint32_t l01 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u);
+      const uint32_t h01 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
+      const uint32_t l23 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
+      const uint32_t h23 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
+      uint32_t* d = cols + (16 * q + 4 * c) * 64 + lane;
+      d[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+      d[64] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+      d[128] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+      d[192] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+    }
+  }
+  if (tid < 64) cols[S * 64 + tid] = 0u;
+  // sums: VT: pair p = m * threads + tid = (row p % 256, class p / 256);
+  // else wave's class slot m, rows lane + 64 j at [4 m + j]
+  float acc[kColsMaxAcc];
+#pragma unroll
+  for (int m = 0; m < kColsMaxAcc; ++m) {
+    const int p = m * (int)blockDim.x + tid;
+    const int64_t r = VT ? row0 + (p & 255) : row0 + lane + 64 * (m & 3);
+    const int k = VT ? p >> 8 : wave + (m >> 2) * nw;
+    acc[m] = (k < K && r < n) ? out[r * K + k] : 0.0f;
+  }
+  const uint8_t* cols8 = reinterpret_cast<const uint8_t*>(cols);
+  const uint32_t lane4 = (uint32_t)lane * 4u;
+  // the values of tree t (table at LDS words tb) for the lane's four rows
+  auto walk = [&](int t, const uint32_t* tb, float (&v)[4]) {
+    const uint32_t* __restrict__ u = uni + (int64_t)t * kColsUni;
+    uint32_t s[15];
+#pragma unroll
+    for (int i = 0; i < 15; ++i) {
+      const uint32_t w = (u[i >> 1] >> (16 * (i & 1))) & 0xffffu;
+      const uint32_t c = *reinterpret_cast<const uint32_t*>(cols8 + (((w >> 7) << 8) + lane4));
+      s[i] = c + (w & 0x7fu) * 0x01010101u;
+    }
+    // bit 7 of each byte: the way at level 0, 1, 2, 3 of that row's path
+    const uint32_t s0 = s[0];
+    const uint32_t s1 = bit_select(s0, s[2], s[1]);
+    const uint32_t s2 = bit_select(s0, bit_select(s1, s[6], s[5]), bit_select(s1, s[4], s[3]));
+    const uint32_t s3 = bit_select(
+        s0,
+        bit_select(s1, bit_select(s2, s[14], s[13]), bit_select(s2, s[12], s[11])),
+        bit_select(s1, bit_select(s2, s[10], s[9]), bit_select(s2, s[8], s[7])));
+    // heap index 16 + path of each row, one byte each
+    const uint32_t g4 = 0x10101010u | ((s0 & kBit7) >> 4) | ((s1 & kBit7) >> 5) |
+                        ((s2 & kBit7) >> 6) | ((s3 & kBit7) >> 7);
+    uint32_t g[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) g[j] = (g4 >> (8 * j)) & 0xffu;
+    for (int d = kColsTop; d < DX; ++d) {
+      uint32_t w[4], c[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = tb[(int)g[j] - (1 << kColsTop)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[j] = cols8[(w[j] & 0xffffff00u) | (lane4 + (uint32_t)j)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) g[j] = 2u * g[j] + (c[j] > (w[j] & 0xffu) ? 1u : 0u);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(tb[(int)g[j] - (1 << kColsTop)]);
+  };
+  for (int t0 = 0; t0 < T; t0 += TC) {
+    const int tc = T - t0 < TC ? T - t0 : TC;
+    __syncthreads();  // columns staged / the previous chunk's tables done with
+    {
+      const u4* src = reinterpret_cast<const u4*>(tab + (int64_t)t0 * GW);  // GW % 4 == 0
+      u4* dst = reinterpret_cast<u4*>(tabs);
+      for (int i = tid; i < tc * GW / 4; i += blockDim.x) dst[i] = src[i];
+    }
+    __syncthreads();
+    if constexpr (VT) {
+      for (int j = wave; j < tc; j += nw) {
+        float v[4];
+        walk(t0 + j, tabs + j * GW, v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vals[j * kColsRows + lane + 64 * i] = v[i];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < kColsMaxAcc; ++m) {
+        const int p = m * (int)blockDim.x + tid;
+        const int k = p >> 8;
+        if (k < K) {  // (t0 is a multiple of K)
+          float a = acc[m];
+          for (int j = k; j < tc; j += K) a = a + vals[j * kColsRows + (p & 255)];
+          acc[m] = a;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < kColsMaxAcc / 4; ++m) {
+        for (int j = wave + m * nw; j < tc && wave + m * nw < K; j += K) {
+          float v[4];
+          walk(t0 + j, tabs + j * GW, v);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[4 * m + i] = acc[4 * m + i] + v[i];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < kColsMaxAcc; ++m) {
+    const int p = m * (int)blockDim.x + tid;
+    const int64_t r = VT ? row0 + (p & 255) : row0 + lane + 64 * (m & 3);
+    const int k = VT ? p >> 8 : wave + (m >> 2) * nw;
+    if (k < K && r < n) out[r * K + k] = acc[m];
+  }
+}
+template __global__ void predict_cols_kernel<false>(const int8_t*, int64_t, int64_t, int32_t,
+                                                    const uint32_t*, const uint32_t*, int32_t,
+                                                    int32_t, int32_t, int32_t, float*,
+                                                    const int32_t*);
+template __global__ void predict_cols_kernel<true>(const int8_t*, int64_t, int64_t, int32_t,
+                                                   const uint32_t*, const uint32_t*, int32_t,
+                                                   int32_t, int32_t, int32_t, float*,
+                                                   const int32_t*);
+
+// block shape of predict_cols_kernel: waves, trees per chunk, whether values go
+// through LDS; 0 when a chunk of one round does not fit
+int predict_cols_plan(int64_t S, int32_t K, int32_t D, int32_t n_rounds, int32_t* DX_out,
+                      int32_t* waves_out, int32_t* TC_out, bool* vt_out, size_t* lds_out) {
+  const int32_t DX = std::max(D, kColsTop);
+  if (S % 16 != 0 || DX > 8 || S > 511) return 0;
+  const int64_t GW = (int64_t(2) << DX) - (1 << kColsTop);
+  const bool vt = K < 8;
+  if (K > 16 * (kColsMaxAcc / 4)) return 0;
+  const int64_t colb = (S + 1) * 256, per = 4 * GW + (vt ? 4 * kColsRows : 0);
+  // tables of about 24 KB (48 KB with values) a chunk, in whole rounds
+  int64_t rounds = std::max<int64_t>(1, (vt ? 48 : 24) * 1024 / (per * K));
+  rounds = std::min<int64_t>(rounds, n_rounds);
+  while (rounds > 1 && colb + rounds * K * per > 156 * 1024) --rounds;
+  const int64_t lds = colb + rounds * K * per;
+  if (lds > 156 * 1024) return 0;
+  // waves: a class each, or 16 sharing the trees
+  int32_t waves = 16;
+  if (!vt) {
+    const int32_t per_wave = (K + 15) / 16;
+    waves = (K + per_wave - 1) / per_wave;
+  }
+  *DX_out = DX;
+  *waves_out = waves;
+  *TC_out = (int32_t)(rounds * K);
+  *vt_out = vt;
+  *lds_out = (size_t)lds;
+  return 1;
+}
+
+// in-place row softmax over K logits: exp(x - max) / sum, sequential in k
+// (up to kSoftmaxLds classes: a workgroup's 256 rows are one contiguous run,
+// moved through LDS with coalesced loads and stores; a thread per row straight
+// from memory touches 64 lines per load and read each row three times: 83 ->
+// 26 us for 1M rows of 10 classes)
+__global__ __launch_bounds__(256) void softmax_rows_kernel(float* __restrict__ x, int64_t n,
+                                                           int32_t K) {
+  extern __shared__ float xs[];  // [256][K | 1], staged rows
+  const int64_t i0 = (int64_t)blockIdx.x * 256;
+  const int64_t i = i0 + threadIdx.x;
+  const bool staged = K <= kSoftmaxLds;
+  const int ks = K | 1;  // odd: the rows of a wave start in different banks
+  const int64_t left = n - i0;
+  const int words = (int)(left < 256 ? left : 256) * K;
+  if (staged) {
+    for (int w = threadIdx.x; w < words; w += 256) xs[w / K * ks + w % K] = x[i0 * K + w];
+    __syncthreads();
+  }
+  if (i < n) {
+    float* r = staged ? xs + threadIdx.x * ks : x + i * K;
+    float m = r[0];
+    for (int k = 1; k < K; ++k) m = r[k] > m ? r[k] : m;
+    float s = 0.0f;
+    for (int k = 0; k < K; ++k) {
+      const float e = wgbm_expf(r[k] - m);
+      r[k] = e;
+      s = s + e;
+    }
+    for (int k = 0; k < K; ++k) r[k] = r[k] / s;
+  }
+  if (staged) {
+    __syncthreads();
+    for (int w = threadIdx.x; w < words; w += 256) x[i0 * K + w] = xs[w / K * ks + w % K];
+  }
 }
 
 // ---------------------------------------------------------------------------
