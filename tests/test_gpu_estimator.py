@@ -572,6 +572,37 @@ def test_chunked_levels_regression_bit_exact(gpu, level_bytes):
     assert np.array_equal(bits(m.predict(X)), bits(ref.predict_codes(codes)))
 
 
+@pytest.mark.parametrize("N,F,B,depth,classes", [
+    (41, 3, 5, 3, 0), (1023, 20, 32, 5, 0), (1025, 30, 127, 7, 0), (4097, 512, 10, 3, 0),
+    (4097, 513, 10, 3, 0), (8193, 33, 63, 7, 3), (16_384, 40, 2, 6, 0), (16_385, 40, 16, 4, 0),
+    (12_289, 17, 9, 10, 0)])
+def test_one_launch_levels_equal_level_chain(gpu, N, F, B, depth, classes):
+    """One-era rounds of few rows (one launch per level) grow the level chain's
+    trees: rows-per-thread remainders, the row and (feature, tree) limits, deep
+    trees with early leaves, class trees, codes outside the bins, residuals of
+    very different scales (nodes with shifts of their own), a feature subset."""
+    print_case("estimator", "one launch per level", N, F, B, depth, classes)
+    rng = np.random.default_rng(N + B)
+    X = rng.integers(0, B, (N, F)).astype(np.int8)
+    X[rng.random((N, F)) < 0.01] = -1
+    y = X[:, 0] / B + 0.3 * rng.standard_normal(N)
+    kw = dict(num_bins=B, max_depth=depth, n_estimators=3, learning_rate=0.5, min_child_weight=3)
+    if classes:
+        kw["objective"] = "multiclass"
+        y = np.digitize(y, np.quantile(y, [0.4, 0.7]))
+    else:
+        y = np.where(X[:, 1] == 0, 1e5 * y, 1e-3 * y).astype(F32)
+    fits = []
+    for key8 in (1, 0):
+        m = WarpGBM(colsample_bytree=0.9 if F < 512 else 1.0, random_state=1, **kw)
+        m._engine_tuning = {8: key8}
+        fits.append(m.fit(X, y))
+    a, b = fits
+    assert a.forest == b.forest
+    assert sum(str(t).count("'feature'") for t in a.forest) > 0
+    assert np.array_equal(bits(a.per_era_feature_importance_), bits(b.per_era_feature_importance_))
+
+
 def test_chunked_levels_multiclass_and_eras_bit_exact(gpu):
     print_case("estimator", "chunked levels multiclass / DES direct / large eras")
     # softmax, 4 class trees per round: chunks of nodes across trees

@@ -131,6 +131,14 @@ __device__ inline int node_shift_rule(uint32_t absmax_bits, int parent_shift,
   const int s_own = wgbm_shift_from_absmax(__uint_as_float(absmax_bits), qbits);
   return s_own - parent_shift >= kNodeShiftStep ? s_own : parent_shift;
 }
+// A leaf's value from the exact sum of its rows' wide quantisation (two
+// words, see finish_node) and their count.
+__device__ inline float leaf_mean(int64_t qh, int64_t ql, int64_t count, int32_t s63) {
+  const int64_t hi = qh + (ql >> 32);
+  const int64_t lo = ql & 0xffffffffll;
+  const double sum = (double)hi * 4294967296.0 + (double)lo;
+  return (float)(ldexp(sum, -s63) / (double)count);
+}
 // Several eras: the histogram shift of one (node, era) segment from the
 // float bits of its largest |residual| (0 for an empty, all-zero or
 // non-finite segment)
@@ -413,6 +421,43 @@ __global__ void predict_heap_kernel(const int8_t* codes, int64_t n, int64_t S, i
 __global__ void complete_tables_kernel(const int32_t* feat, const int32_t* bin, const float* leaf,
                                        int64_t T, int32_t D, int64_t S, float lr,
                                        uint32_t* cnode, float* cleaf);
+// one-era rounds of few rows, one launch per level (engine_small.hip): word
+// arrays [T * H] by heap index; ids: heap index of every row
+constexpr int64_t kSmallMaxRows = 16384;
+// (feature, tree) workgroups a launch may have: two on each CU at once; with
+// more, every level takes that many rounds of them.  Us per round, level chain
+// / one launch per level: 10000 rows x 50, depth 5 177 / 76; 16000 x 200 227 /
+// 106; 16000 x 500 241 / 179; 10000 x 50, 10 classes, depth 6 236 / 162; 16000 x
+// 100, 3 classes, 127 bins 497 / 279; past it 10000 x 100, 10 classes 261 / 287;
+// 16000 x 1000 248 / 314.
+constexpr int64_t kSmallMaxWork = 512;
+struct SmallArgs {
+  int64_t n;
+  int32_t B, H, depth, max_depth, n_feat_wg, n_part, from_target, qbits, s63_add;
+  int32_t hist_copies_log2, max_copies_log2, tot_copies_log2;
+  float mcw, eps, msg, lr;
+  const int8_t* codes_cm;
+  const int32_t* feat_sel;
+  const float* target;       // from_target: the root level computes the residuals
+  float* pred;
+  int64_t pcol;
+  const float* resid;        // [T][n]
+  float* resid_out;
+  const uint32_t* abs_part;  // [T][n_part] maxima (root level, not from_target)
+  uint32_t* absmax;
+  int32_t* shifts;
+  const uint16_t* ids_in;
+  uint16_t* ids_out;
+  unsigned long long* best;
+  int32_t* node_shift;
+  int32_t* present;
+  int64_t* tot_qh;
+  int64_t* tot_ql;
+  int64_t* tot_c;
+  TreeRecord rec;
+};
+bool small_round_fits(int64_t n, int32_t F, int32_t B, int32_t max_depth);
+int launch_small_level(SmallArgs a, int T, hipStream_t st);
 // column-block predictor: top levels evaluated whole, their words per tree
 // (padded), (row, class) sums per thread, rows per workgroup
 constexpr int kSoftmaxLds = 32;  // classes of a row softmax staged in LDS (33 KB)

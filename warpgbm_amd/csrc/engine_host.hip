@@ -117,6 +117,16 @@ struct Engine {
   float* leaf_val = nullptr;
   unsigned long long* best = nullptr;  // packed split picks, two depths (parity)
   int64_t pick_stride = 0;             // words per depth in best / agree_max
+  // one era and few rows: rounds of one launch per level (engine_small.hip);
+  // off when a knob of the level chain is set
+  bool small_fits = false;
+  int small_on = 1;
+  struct {
+    uint16_t* ids[2];
+    unsigned long long* best;
+    int32_t *node_shift, *present;
+    int64_t *tot_qh, *tot_ql, *tot_c;
+  } sr{};
   std::vector<void*> allocs;
   // one allocation for the buffers sized at creation (hipMalloc and hipFree
   // cost ~5 and ~20 us each here: ~60 buffers took ~1.5 ms per fit)
@@ -234,7 +244,9 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
     // the chosen split's per-era gains; the pair codes; 64 MiB of slack
     const int64_t keys = e->n_keys_max, tn = T * nodes_max;
     const int64_t pcodes = (e->des_direct && B <= 7) ? N * pair_stride((int32_t)F) : 0;
-    const int64_t need = e->nc_max * per_node + T * N * 29 + keys * 132 + tn * 76 + tn * E * 4 +
+    const int64_t small =
+        E == 1 && small_round_fits(N, (int32_t)F, (int32_t)B, D) ? T * N * 4 + T * e->H * 40 : 0;
+    const int64_t need = small + e->nc_max * per_node + T * N * 29 + keys * 132 + tn * 76 + tn * E * 4 +
                          pcodes + ((int64_t)64 << 20);
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && (size_t)need > free_b) {
@@ -349,11 +361,35 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
       return (int)err;
     }
   }
+  e->small_fits = E == 1 && small_round_fits(N, (int32_t)F, (int32_t)B, D);
+  if (e->small_fits) {
+    const int64_t W = T * e->H;
+    for (int k = 0; k < 2; ++k) E_ALLOC(e->sr.ids[k], T * N);
+    E_ALLOC(e->sr.best, W);
+    E_ALLOC(e->sr.node_shift, W);
+    E_ALLOC(e->sr.present, W);
+    E_ALLOC(e->sr.tot_qh, W);
+    E_ALLOC(e->sr.tot_ql, W);
+    E_ALLOC(e->sr.tot_c, W);
+    const hipError_t err = hipMemset(e->sr.best, 0, sizeof(unsigned long long) * (size_t)W);
+    if (err != hipSuccess) {
+      wgbm_set_error("engine: clearing the split picks failed: %s", hipGetErrorString(err));
+      engine_destroy(e);
+      return (int)err;
+    }
+  }
   *out = e;
   return 0;
 }
 
 int engine_set_tuning(Engine* e, int key, int64_t value) {
+  if (key == 8) {
+    WGBM_REQUIRE(value == 0 || value == 1, "one launch per level must be 0 or 1");
+    e->small_on = (int)value;
+    return 0;
+  }
+  // the other knobs choose parts of the level chain
+  if (key >= 1 && key <= 7) e->small_on = 0;
   if (key == 1) {
     WGBM_REQUIRE(value == 0 || (value >= 256 && value <= WGBM_MAX_TILE_ROWS),
                  "hist tile rows must be 0 or in [256, %d]", WGBM_MAX_TILE_ROWS);
@@ -562,6 +598,58 @@ static HistLaunch level_hist(const Engine* e, int cur, int64_t k0) {
 
 static inline unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
+// a one-era round of few rows: residuals (regression: in the root level's
+// launch), then one launch per level
+static int small_round(Engine* e, const void* target, float* pred, const int32_t* feat_sel,
+                       int32_t n_sel, const TreeRecord& rec, hipStream_t st) {
+  const EngineConfig& c = e->c;
+  const int T = c.n_trees, D = c.max_depth;
+  SmallArgs a{};
+  a.n = c.n_rows;
+  a.B = c.num_bins;
+  a.H = e->H;
+  a.max_depth = D;
+  a.qbits = e->qbits;
+  a.s63_add = 62 - e->qbits;
+  a.mcw = c.min_child_weight;
+  a.eps = c.l2_reg;
+  a.msg = c.min_split_gain;
+  a.lr = c.learning_rate;
+  a.codes_cm = c.codes_cm;
+  a.feat_sel = feat_sel;
+  a.pred = pred;
+  a.pcol = c.objective == 0 ? 0 : c.n_rows;
+  a.resid = a.resid_out = e->resid;
+  a.absmax = e->absmax;
+  a.shifts = e->shifts;
+  a.best = e->sr.best;
+  a.node_shift = e->sr.node_shift;
+  a.present = e->sr.present;
+  a.tot_qh = e->sr.tot_qh;
+  a.tot_ql = e->sr.tot_ql;
+  a.tot_c = e->sr.tot_c;
+  a.rec = rec;
+  if (c.objective == 1) {
+    const int nres = (int)std::min<int64_t>(blocks_for(c.n_rows, 256), kResidBlocks);
+    hipLaunchKernelGGL(residual_softmax_kernel, dim3(nres), dim3(256), 0, st, pred,
+                       (const int32_t*)target, c.n_rows, T, e->resid, e->abs_part);
+    WGBM_LAUNCH_CHECK();
+    a.abs_part = e->abs_part;
+    a.n_part = nres;
+  }
+  for (int d = 0; d <= D; ++d) {
+    a.depth = d;
+    a.from_target = d == 0 && c.objective == 0;
+    a.target = (const float*)target;
+    a.n_feat_wg = d < D ? n_sel : 0;
+    a.ids_in = e->sr.ids[(d & 1) ^ 1];
+    a.ids_out = e->sr.ids[d & 1];
+    const int r = launch_small_level(a, T, st);
+    if (r) return r;
+  }
+  return 0;
+}
+
 int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat_sel,
                  int32_t n_sel, const TreeRecord& rec, hipStream_t st) {
   const EngineConfig& c = e->c;
@@ -570,6 +658,8 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
   WGBM_REQUIRE(rec.H == e->H, "engine_round: record has H=%d, expected %d", rec.H, e->H);
   const int T = c.n_trees, E = c.num_eras, F = c.n_feats, B = c.num_bins, D = c.max_depth;
   const int64_t N = c.n_rows;
+  if (e->small_fits && e->small_on && (int64_t)T * n_sel <= kSmallMaxWork)
+    return small_round(e, target, pred, feat_sel, n_sel, rec, st);
   if (!e->part) {
     const int r = presize_levels(e);
     if (r) return r;

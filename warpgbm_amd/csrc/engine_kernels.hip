@@ -344,10 +344,7 @@ __device__ inline void finish_node(
       rec.leaf[h] = 0.0f;
       nroute[tn] = NodeRoute{col, b, 0.0f, s63};
     } else {
-      const int64_t hi = sqh + (sql >> 32);
-      const int64_t lo = sql & 0xffffffffll;
-      const double sum = (double)hi * 4294967296.0 + (double)lo;
-      const float v = (float)(ldexp(sum, -s63) / (double)sc);
+      const float v = leaf_mean(sqh, sql, sc, s63);
       leaf_val[tn] = v;
       rec.feat[h] = -1;
       rec.bin[h] = -1;
