@@ -192,6 +192,15 @@ __device__ __forceinline__ void wgbm_lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Order between a wave's own agent-scope atomics: what it stored with them
+// before this has reached the agent's point of coherence before any memory
+// operation after it.  Enough to hand over data that is both written and read
+// with agent-scope atomics (they bypass the XCDs' L2s); a __threadfence would
+// also write back every dirty line of this XCD's L2.
+__device__ __forceinline__ void wgbm_atomics_done() {
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // A 64-bit value of one lane (lane wave-uniform).
 __device__ __forceinline__ int64_t wgbm_readlane_i64(int64_t x, int lane) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)x, lane);

@@ -1813,11 +1813,11 @@ __global__ __launch_bounds__(256) void split_finish_e1_kernel(
   if (bpn > 1) {
     if (threadIdx.x == 0) {
       if (k) atomicMax(best + tn, k);
-      __threadfence();  // the key is visible before the arrival is counted
+      wgbm_atomics_done();  // the key is visible before the arrival is counted
       const uint32_t prev = atomicAdd(done + tn, 1u);
       const bool last = prev == (uint32_t)(bpn - 1);
+      wgbm_atomics_done();  // the pick is read after the count
       if (last) {
-        __threadfence();  // every other workgroup's key is visible
         k = __hip_atomic_load(best + tn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         done[tn] = 0u;    // ready for the next level
       }
