@@ -229,7 +229,8 @@ __global__ void level_scan_kernel(int32_t nb, PartSums ps, int32_t T, int32_t no
                                   int64_t n_pos, const int64_t* seg, const int32_t* present,
                                   const int32_t* split_l, LevelNext nx, int32_t n_list,
                                   int32_t tile_rows, int32_t max_tiles, Tile* tiles,
-                                  int32_t* key_tile_start, int32_t* n_tiles);
+                                  int32_t* key_tile_start, int32_t* n_tiles,
+                                  int32_t plan_present, float mcw);
 // One-era split levels in one pass: route, rank and place every position
 // (route_kernel + scatter_kernel without the block prefix between them), for
 // levels of at most kPartition1MaxNodes (tree, node)s.
@@ -338,13 +339,14 @@ __global__ void des_alive_kernel(const int64_t* seg, int32_t E, int32_t n_tn, fl
 __global__ void des_block_kernel(const float* gain, const int8_t* dir, int32_t E, int32_t n_tn,
                                  int64_t ncand, const int32_t* present, const uint32_t* alive,
                                  double* bsum, int8_t* bdir);
+template <bool ONE_BLOCK>
 __global__ void des_combine_pick_kernel(const double* bsum, const int8_t* bdir, int32_t E,
                                         int32_t n_tn, int64_t ncand, const int32_t* present,
                                         const uint32_t* alive, float min_split_gain,
                                         int32_t* wg_agree, unsigned long long* wg_key,
                                         unsigned long long* best, uint32_t* done,
-                                        const float* staged, const int64_t* seg, float mcw,
-                                        int32_t nb, int32_t n_sel, int32_t* split_l,
+                                        const float* staged, const int8_t* sdir, const int64_t* seg,
+                                        float mcw, int32_t nb, int32_t n_sel, int32_t* split_l,
                                         int32_t* split_b, float* split_gain_era);
 __global__ void local_scatter_kernel(const int32_t* feat_sel, int32_t n_sel, int32_t F,
                                      int32_t* local_of);

@@ -797,11 +797,13 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
           LevelPlan lp;
           r = era_tile_plan(e, nc, (n_tn + nc - 1) / nc, &lp);
           if (r) return r;
-          hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
-                             (int64_t)0, lp.n_list, (const int32_t*)nullptr, (int32_t)lp.R, 0,
-                             (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
-                             e->present[cur] + c0, E, mcw);
-          WGBM_LAUNCH_CHECK();
+          if (!planned) {  // (else by the previous level's scan)
+            hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
+                               (int64_t)0, lp.n_list, (const int32_t*)nullptr, (int32_t)lp.R, 0,
+                               (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
+                               e->present[cur] + c0, E, mcw);
+            WGBM_LAUNCH_CHECK();
+          }
           HistLaunch a = level_hist(e, cur, k0);
           a.tiles = e->htiles;
           a.n_tiles = e->hn;
@@ -826,25 +828,29 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
           tm = timer_begin(tag);
           if (tm) WGBM_CHECK(hipEventRecord(timer_start_event(tm), st));
         }
-        if (!(alive_ready && nc == n_tn)) {
-          hipLaunchKernelGGL(des_alive_kernel, dim3(blocks_for((int64_t)nc * W, 256)), dim3(256),
-                             0, st, e->seg[cur] + k0, E, nc, mcw, e->alive);
+        const bool one_block = E <= kDesEraBlock;
+        if (!one_block) {
+          if (!(alive_ready && nc == n_tn)) {
+            hipLaunchKernelGGL(des_alive_kernel, dim3(blocks_for((int64_t)nc * W, 256)),
+                               dim3(256), 0, st, e->seg[cur] + k0, E, nc, mcw, e->alive);
+            WGBM_LAUNCH_CHECK();
+          }
+          hipLaunchKernelGGL(des_block_kernel,
+                             dim3(blocks_for((int64_t)nc * W * ((ncand + 63) / 64) * 64, 256)),
+                             dim3(256), 0, st, e->sgain, e->sdir, E, nc, ncand,
+                             e->present[cur] + c0, e->alive, e->bsum, e->bdir);
           WGBM_LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL(des_block_kernel,
-                           dim3(blocks_for((int64_t)nc * W * ((ncand + 63) / 64) * 64, 256)),
-                           dim3(256), 0, st, e->sgain, e->sdir, E, nc, ncand,
-                           e->present[cur] + c0, e->alive, e->bsum, e->bdir);
-        WGBM_LAUNCH_CHECK();
         // block sums in block order, the pick and the record in one launch
         // (the last workgroup of each node picks from the workgroups'
         // summaries and finishes the node)
-        hipLaunchKernelGGL(des_combine_pick_kernel,
+        hipLaunchKernelGGL((one_block ? des_combine_pick_kernel<true>
+                                      : des_combine_pick_kernel<false>),
                            dim3((unsigned)((int64_t)nc * ((ncand + 255) / 256))), dim3(256), 0,
                            st, e->bsum, e->bdir, E, nc, ncand, e->present[cur] + c0, e->alive,
                            msg, e->wg_agree, e->wg_key, best + c0, e->done + c0, e->sgain,
-                           e->seg[cur] + k0, mcw, (int32_t)(B - 1), n_sel, e->split_l + c0,
-                           e->split_b + c0, e->split_gain + k0);
+                           e->sdir, e->seg[cur] + k0, mcw, (int32_t)(B - 1), n_sel,
+                           e->split_l + c0, e->split_b + c0, e->split_gain + k0);
         WGBM_LAUNCH_CHECK();
         if (tm) {
           WGBM_CHECK(hipEventRecord(timer_stop_event(tm), st));
@@ -1087,12 +1093,20 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
         WGBM_LAUNCH_CHECK();
         planned = next_hist;
       } else if (n_tn <= kLevelScanMaxNodes) {
+        // (the next era level over tiles, whole: its tiles too)
+        const bool next_tiles = d + 1 < D && e->des_direct && era_level_tiles(e, d + 1) &&
+                                2 * (int64_t)n_tn <= e->nc_max;
+        if (next_tiles) {
+          const int r = era_tile_plan(e, 2 * (int64_t)n_tn, 1, &lp);
+          if (r) return r;
+        }
         hipLaunchKernelGGL(level_scan_kernel, dim3(1), dim3(1024), 0, st, (int32_t)e->nb, e->ps,
                            T, nodes, E, n_pos, e->seg[cur], e->present[cur], e->split_l, nx,
-                           next_hist ? lp.n_list : 0, (int32_t)lp.R, (int32_t)lp.max_tiles,
-                           e->htiles, e->hkts, e->hn);
+                           next_hist || next_tiles ? lp.n_list : 0, (int32_t)lp.R,
+                           (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
+                           next_tiles ? 1 : 0, mcw);
         WGBM_LAUNCH_CHECK();
-        planned = next_hist;
+        planned = next_hist || next_tiles;
       } else {
         hipLaunchKernelGGL(block_scan_kernel, dim3(1), dim3(1024), 0, st, (int32_t)e->nb, e->ps);
         WGBM_LAUNCH_CHECK();

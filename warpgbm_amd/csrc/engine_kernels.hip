@@ -1675,7 +1675,7 @@ __global__ __launch_bounds__(1024) void level_scan_kernel(
     const int64_t* __restrict__ seg, const int32_t* __restrict__ present,
     const int32_t* __restrict__ split_l, LevelNext nx, int32_t n_list, int32_t tile_rows,
     int32_t max_tiles, Tile* __restrict__ tiles, int32_t* __restrict__ key_tile_start,
-    int32_t* __restrict__ n_tiles) {
+    int32_t* __restrict__ n_tiles, int32_t plan_present, float mcw) {
   block_scan_body(nb, ps);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1734,8 +1734,11 @@ __global__ __launch_bounds__(1024) void level_scan_kernel(
   }
   if (n_list <= 0) return;  // uniform
   __syncthreads();
-  plan_tiles_body(nx.seg_next, 0, n_list, nx.key_list_next, tile_rows, 0, max_tiles, tiles,
-                  key_tile_start, n_tiles);
+  // plan_present: the tiles of every live segment of the next level (the era
+  // levels of few large segments), else those of its key list
+  plan_tiles_body(nx.seg_next, 0, n_list, plan_present ? nullptr : nx.key_list_next, tile_rows, 0,
+                  max_tiles, tiles, key_tile_start, n_tiles,
+                  plan_present ? nx.present_next : nullptr, E, mcw);
 }
 
 // One-era split search fused with the leaf / record step: one lane per

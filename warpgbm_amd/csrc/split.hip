@@ -909,13 +909,18 @@ __global__ __launch_bounds__(256) void des_block_kernel(
 // summaries, stores the pick to best[tn], resets done[tn], and writes
 // split_l / split_b and the chosen split's staged gain of every era (0 for
 // a dead segment), as des_finish_kernel.
+// ONE_BLOCK (at most 32 eras: one block): the era sums are made here, from the
+// staged gains and directions in era order (bsum, bdir and alive are not used),
+// which saves des_block_kernel's and des_alive_kernel's launches.
+template <bool ONE_BLOCK>
 __global__ __launch_bounds__(256) void des_combine_pick_kernel(
     const double* __restrict__ bsum, const int8_t* __restrict__ bdir, int32_t E, int32_t n_tn,
     int64_t ncand, const int32_t* __restrict__ present, const uint32_t* __restrict__ alive,
     float min_split_gain, int32_t* __restrict__ wg_agree, unsigned long long* __restrict__ wg_key,
     unsigned long long* __restrict__ best, uint32_t* __restrict__ done,
-    const float* __restrict__ staged, const int64_t* __restrict__ seg, float mcw, int32_t nb,
-    int32_t n_sel, int32_t* __restrict__ split_l, int32_t* __restrict__ split_b,
+    const float* __restrict__ staged, const int8_t* __restrict__ sdir,
+    const int64_t* __restrict__ seg, float mcw, int32_t nb, int32_t n_sel,
+    int32_t* __restrict__ split_l, int32_t* __restrict__ split_b,
     float* __restrict__ split_gain_era) {
   __shared__ int s_a[4];
   __shared__ unsigned long long s_k[4];
@@ -933,10 +938,45 @@ __global__ __launch_bounds__(256) void des_combine_pick_kernel(
     }
     return;
   }
-  const uint32_t* al = alive + (int64_t)tn * W;
+  const uint32_t* al = ONE_BLOCK ? nullptr : alive + (int64_t)tn * W;
   int a = -1;
   float cr = 0.0f;
-  if (c < ncand) {
+  if constexpr (ONE_BLOCK) {
+    // the eras that can hold a split, as des_alive_kernel
+    bool live = false;
+    if (lane < E) {
+      const int64_t k0 = (int64_t)tn * E;
+      live = !des_segment_dead(seg[k0 + lane + 1] - seg[k0 + lane], mcw);
+    }
+    const uint32_t m = (uint32_t)__ballot(live);
+    const int64_t c64 = (ncand + 63) / 64;
+    const int64_t o = des_stage_slot(tn, 0, W, c64, c < ncand ? c : ncand - 1);
+    double acc = 0.0;
+    int ds = 0;
+    constexpr int G = 8;  // eras whose loads are issued together (slots of a
+                          // block exist up to era 31; a dead one's is not added)
+    for (int e0 = 0; e0 < E; e0 += G) {
+      if (((m >> e0) & 0xffu) == 0u) continue;  // uniform
+      float g[G];
+      int dv[G];
+#pragma unroll
+      for (int k = 0; k < G; ++k) {
+        g[k] = staged[o + (e0 + k) * 64];
+        dv[k] = (int)sdir[o + (e0 + k) * 64];
+      }
+#pragma unroll
+      for (int k = 0; k < G; ++k) {
+        if ((m >> (e0 + k)) & 1u) {
+          acc += (double)g[k];  // era order
+          ds += dv[k];
+        }
+      }
+    }
+    if (c < ncand) {
+      cr = (float)(acc / (double)E);
+      a = ds < 0 ? -ds : ds;
+    }
+  } else if (c < ncand) {
     double acc = 0.0;
     int ds = 0;
     // blocks in groups of 8, the group's loads issued together (a block
@@ -1059,6 +1099,15 @@ __global__ __launch_bounds__(256) void des_combine_pick_kernel(
                              : staged[des_stage_slot(tn, e, W, c64, idx)];
   }
 }
+
+template __global__ void des_combine_pick_kernel<false>(
+    const double*, const int8_t*, int32_t, int32_t, int64_t, const int32_t*, const uint32_t*,
+    float, int32_t*, unsigned long long*, unsigned long long*, uint32_t*, const float*,
+    const int8_t*, const int64_t*, float, int32_t, int32_t, int32_t*, int32_t*, float*);
+template __global__ void des_combine_pick_kernel<true>(
+    const double*, const int8_t*, int32_t, int32_t, int64_t, const int32_t*, const uint32_t*,
+    float, int32_t*, unsigned long long*, unsigned long long*, uint32_t*, const float*,
+    const int8_t*, const int64_t*, float, int32_t, int32_t, int32_t*, int32_t*, float*);
 
 // local index of every feature of the round's subset (local_of is -1 elsewhere)
 __global__ void local_scatter_kernel(const int32_t* __restrict__ feat_sel, int32_t n_sel,
