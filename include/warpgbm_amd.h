@@ -288,7 +288,7 @@ int wgbm_engine_round(wgbm_engine* eng, const void* target, float* pred, const i
  * scatter); key 7 = the era levels' partition (1 = the route reserves each
  * (node, era) segment's child ranges and leaves its sums for the node scan,
  * no block prefix, default; 0 = route, block prefix, node scan, scatter);
- * key 8 = one-era rounds of at most 16384 rows and 512 (feature, tree)s (1 =
+ * key 8 = one-era rounds of at most 20480 rows and 512 (feature, tree)s (1 =
  * one launch per level, default; 0 = the level chain; setting any of keys 1
  * to 7 takes the level chain too, whose parts they choose).
  * Set before the first round; every setting grows the same trees. */

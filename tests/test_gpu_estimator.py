@@ -574,7 +574,7 @@ def test_chunked_levels_regression_bit_exact(gpu, level_bytes):
 
 @pytest.mark.parametrize("N,F,B,depth,classes", [
     (41, 3, 5, 3, 0), (1023, 20, 32, 5, 0), (1025, 30, 127, 7, 0), (4097, 512, 10, 3, 0),
-    (4097, 513, 10, 3, 0), (8193, 33, 63, 7, 3), (16_384, 40, 2, 6, 0), (16_385, 40, 16, 4, 0),
+    (4097, 513, 10, 3, 0), (8193, 33, 63, 7, 3), (16_384, 40, 2, 6, 0), (20_480, 40, 16, 4, 0), (20_481, 9, 16, 4, 0),
     (12_289, 17, 9, 10, 0)])
 def test_one_launch_levels_equal_level_chain(gpu, N, F, B, depth, classes):
     """One-era rounds of few rows (one launch per level) grow the level chain's

@@ -425,11 +425,11 @@ __global__ void complete_tables_kernel(const int32_t* feat, const int32_t* bin, 
                                        uint32_t* cnode, float* cleaf);
 // one-era rounds of few rows, one launch per level (engine_small.hip): word
 // arrays [T * H] by heap index; ids: heap index of every row
-constexpr int64_t kSmallMaxRows = 16384;
+constexpr int64_t kSmallMaxRows = 20480;
 // (feature, tree) workgroups a launch may have: two on each CU at once; with
 // more, every level takes that many rounds of them.  Us per round, level chain
-// / one launch per level: 10000 rows x 50, depth 5 177 / 76; 16000 x 200 227 /
-// 106; 16000 x 500 241 / 179; 10000 x 50, 10 classes, depth 6 236 / 162; 16000 x
+// / one launch per level: 10000 rows x 50, depth 5 177 / 67; 20000 x 50 191 / 96;
+// 16000 x 200 227 / 106; 16000 x 500 241 / 179; 10000 x 50, 10 classes, depth 6 236 / 162; 16000 x
 // 100, 3 classes, 127 bins 497 / 279; past it 10000 x 100, 10 classes 261 / 287;
 // 16000 x 1000 248 / 314.
 constexpr int64_t kSmallMaxWork = 512;
