@@ -171,6 +171,8 @@ void engine_destroy(Engine* e) {
   delete e;
 }
 
+static int presize_levels(Engine* e);
+
 int engine_create(Engine** out, const EngineConfig& cfg) {
   WGBM_REQUIRE(cfg.n_rows > 0 && cfg.n_rows < (int64_t(1) << 31), "engine: n_rows out of range");
   WGBM_REQUIRE(cfg.n_feats > 0, "engine: n_feats must be positive");
@@ -378,6 +380,15 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
       return (int)err;
     }
   }
+  if (e->des_direct) {
+    // here and not in the first round, which allocates nothing on this path
+    // (a stream under capture takes no allocation)
+    const int r = presize_levels(e);
+    if (r) {
+      engine_destroy(e);
+      return r;
+    }
+  }
   *out = e;
   return 0;
 }
@@ -531,9 +542,10 @@ static bool era_level_tiles(const Engine* e, int d) {
   return e->c.n_rows >= rows * (int64_t(1) << d) * e->c.num_eras;
 }
 
-// the tile buffers of every whole level a round histograms, sized once before
-// the first round's launches: growing them level by level would synchronise
-// the device (a buffer in use is freed only after a sync) at each depth
+// the tile buffers of every level a round histograms, sized once, with the
+// engine (direct era path) or before the first round's launches: growing them
+// level by level would synchronise the device (a buffer in use is freed only
+// after a sync) at each depth
 static int presize_levels(Engine* e) {
   int64_t mt = 0;
   if (e->des_direct) {
@@ -660,7 +672,7 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
   const int64_t N = c.n_rows;
   if (e->small_fits && e->small_on && (int64_t)T * n_sel <= kSmallMaxWork)
     return small_round(e, target, pred, feat_sel, n_sel, rec, st);
-  if (!e->part) {
+  if (!e->part && !e->des_direct) {
     const int r = presize_levels(e);
     if (r) return r;
   }
