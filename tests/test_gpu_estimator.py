@@ -603,6 +603,32 @@ def test_one_launch_levels_equal_level_chain(gpu, N, F, B, depth, classes):
     assert np.array_equal(bits(a.per_era_feature_importance_), bits(b.per_era_feature_importance_))
 
 
+@pytest.mark.parametrize("N,F,classes", [(20_481, 3, 0), (102_400, 3, 0), (102_401, 3, 0),
+                                         (204_801, 3, 0), (204_802, 2, 0), (25_600, 1000, 0),
+                                         (34_134, 5, 3)])
+def test_level_tile_rows_bit_exact(gpu, N, F, classes):
+    """Levels with tiles of 512 rows (few workgroups) grow the trees that tiles
+    of 1024 grow, on both sides of the row limit for the root and the levels
+    below it, with one and four feature chunks and with class trees."""
+    print_case("estimator", "tile rows of a level", N, F, classes)
+    rng = np.random.default_rng(N)
+    X = rng.integers(0, 32, (N, F)).astype(np.int8)
+    y = (X[:, 0] / 32 + 0.3 * rng.standard_normal(N)).astype(F32)
+    kw = dict(num_bins=32, max_depth=4, n_estimators=2, learning_rate=0.5, min_child_weight=3)
+    if classes:
+        kw["objective"] = "multiclass"
+        y = np.digitize(y, np.quantile(y, [0.4, 0.7]))
+    fits = []
+    for tuning in ({8: 0}, {1: 1024}):
+        m = WarpGBM(**kw)
+        m._engine_tuning = tuning
+        fits.append(m.fit(X, y))
+    a, b = fits
+    assert a.forest == b.forest
+    assert "'feature'" in str(a.forest[0])
+    assert np.array_equal(bits(a.per_era_feature_importance_), bits(b.per_era_feature_importance_))
+
+
 def test_chunked_levels_multiclass_and_eras_bit_exact(gpu):
     print_case("estimator", "chunked levels multiclass / DES direct / large eras")
     # softmax, 4 class trees per round: chunks of nodes across trees

@@ -442,14 +442,15 @@ int engine_set_tuning(Engine* e, int key, int64_t value) {
   return WGBM_EINVAL;
 }
 
-// histogram tile rows for a level: enough tiles for ~2 workgroups per CU
-static int64_t pick_tile_rows(const Engine* e, int64_t rows_bound) {
+// histogram tile rows for a level: enough tiles for ~2 workgroups per CU, of
+// least rows or more
+static int64_t pick_tile_rows(const Engine* e, int64_t rows_bound, int64_t least = 1024) {
   if (e->hist_tile_rows > 0) return e->hist_tile_rows;
   const int64_t target_wg = kHistTargetWG;
   int64_t tiles = std::max<int64_t>(1, target_wg / e->n_chunks);
   int64_t r = (rows_bound + tiles - 1) / tiles;
   r = (r + 255) / 256 * 256;
-  return std::min<int64_t>(std::max<int64_t>(r, 1024), WGBM_MAX_TILE_ROWS);
+  return std::min<int64_t>(std::max<int64_t>(r, least), WGBM_MAX_TILE_ROWS);
 }
 
 static int ensure_partials(Engine* e, int64_t max_tiles) {
@@ -495,6 +496,17 @@ static int ensure_tiles(Engine* e, int64_t max_tiles) {
   return 0;
 }
 
+// A whole level's tiles have 1024 rows at least (a tile's partial is up to
+// 64 KB, written and read again), 512 where those would give fewer than 100
+// of the 256 CUs a workgroup: the launch then takes as long as one tile's
+// rows, 15 us at 1024.  Us per round with 1024 / 512 / 256 rows: 100003 x 200,
+// 10 bins, depth 3 139 / 126 / 127; 100000 x 100, 32 bins, depth 6 253 / 241 /
+// 249; 50000 x 1000, depth 5 265 / 254 / 273; 40000 x 100, 3 classes 216 / 207
+// / 212; with more workgroups than that 512 rows lose: 50000 x 300, 127 bins
+// (122 workgroups below the root) 484 / 490 / 527; 500000 x 60, 10 bins 234 /
+// 246 / 284.  Era segments keep 1024 (50000 x 100, 3 eras 350 / 355 / 391).
+constexpr int64_t kHistIdleRows = 100 * 1024;
+
 // histogram tiles of level d (the root, or the key pairs of every split: the
 // smaller child, or both children when one takes a finer shift): tile rows,
 // the tile bound, and buffers that hold them
@@ -510,7 +522,8 @@ static void level_plan_sizes(const Engine* e, int d, LevelPlan* lp) {
   // tiles are sized for the smaller children (half the rows); the bound
   // holds the rare level where every split histograms both children
   lp->rows_bound = d == 0 ? T * N : (T * N) / 2;
-  lp->R = pick_tile_rows(e, lp->rows_bound);
+  const bool idle = E == 1 && lp->rows_bound * e->n_chunks <= kHistIdleRows;
+  lp->R = pick_tile_rows(e, lp->rows_bound, idle ? 512 : 1024);
   lp->max_tiles = (T * N) / lp->R + lp->n_list + 1;
 }
 
