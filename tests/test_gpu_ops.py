@@ -423,6 +423,40 @@ def test_predict_heap_paths_bit_exact(gpu, case):
     assert np.array_equal(bits(out.cpu().numpy()), bits(ref))
 
 
+# raw codes, rows, features, classes, rounds, depth: row blocks of the resident
+# predictor (multiples of 64 rows where more fit; one block, a last block of one
+# row, several blocks a workgroup), rows of one 8-byte load, loads per thread in
+# part and in full
+RESIDENT_CASES = [
+    (True, 4096, 8, 1, 30, 5), (True, 4097, 520, 1, 60, 5), (True, 20_001, 1000, 1, 100, 5),
+    (True, 16_449, 1504, 1, 40, 4), (False, 63, 520, 1, 60, 5), (False, 129, 600, 3, 30, 5),
+    (False, 16_385, 1000, 1, 100, 5), (False, 20_003, 640, 10, 12, 4),
+]
+
+
+@pytest.mark.parametrize("case", RESIDENT_CASES, ids=[str(c) for c in RESIDENT_CASES])
+def test_predict_resident_row_blocks_bit_exact(gpu, case):
+    """Trees held in LDS, over raw codes (predict_forest: signed, negative and
+    127 among them) and native ones (predict_heap), against the oracle's walk."""
+    raw_codes, N, F, K, R, depth = case
+    print_case("predict resident", *case)
+    rng = np.random.default_rng(N + F)
+    raw = rng.integers(-2, 35, (N, F)).astype(np.int8)
+    raw[rng.random((N, F)) < 0.01] = 127
+    raw[rng.random((N, F)) < 0.01] = -128
+    feat, binv, leaf, tables = _random_heap(rng, R, K, depth, F, 32)
+    out0 = rng.standard_normal((N, K)).astype(F32)
+    out = t(out0)
+    if raw_codes:
+        padded = np.pad(tables, ((0, 0), (0, 1), (0, 0)))  # 2^(depth + 1) slots
+        node_kernel.predict_forest(t(raw), t(padded), 0.1, out.reshape(-1))
+    else:
+        codes = D.codes_from_int8(D.upload_int8(raw, dev), False, 32)[0]
+        D.predict_heap(codes, t(feat), t(binv), t(leaf), R, K, depth, 0.1, out)
+    ref = clib.predict_tables(raw, tables, F32(0.1), out0, np.tile(np.arange(K, dtype=np.int32), R))
+    assert np.array_equal(bits(out.cpu().numpy()), bits(ref))
+
+
 # rows, features, bins, classes, rounds, depth: the column-block predictor's row
 # blocks (256) and stride groups (16 columns), values through LDS (below 8
 # classes) or sums in registers (one or two classes a wave, to 32), the extension

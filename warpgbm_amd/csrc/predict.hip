@@ -222,14 +222,6 @@ __device__ __forceinline__ uint32_t walk_bytes(uint32_t x, uint32_t bb) {
   return x & ((nz >> 7) * 0xffu);
 }
 
-// Raw int8 codes (the reference's bin_indices, any value) as the walkers
-// read them: a negative code becomes 0, which goes left at every split as the
-// reference's signed `code <= bin` sends it (split bins >= 0); 0..127 stay,
-// so right iff code > bin as there.
-__device__ __forceinline__ uint32_t raw_walk_bytes(uint32_t x) {
-  return x & ~(((x >> 7) & 0x01010101u) * 0xffu);
-}
-
 // A walk over a complete table held in LDS, stepped by LDS byte address: the
 // tree's node words start at `base`, node g (1-based heap index, children 2g
 // and 2g + 1) sits at a = base + 4 (g - 1), so the step to child 2g + x is
@@ -237,6 +229,7 @@ __device__ __forceinline__ uint32_t raw_walk_bytes(uint32_t x) {
 // and the row byte's address per step.
 typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
 typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
+typedef __attribute__((address_space(3))) int8_t lds_i8_t;
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const lds_u8_t*)p;
@@ -252,11 +245,16 @@ struct Walk {
     // select(4, 8) - base, one more instruction per step
     __asm__("" : "+v"(k0), "+v"(k1));
   }
-  // row: LDS address of the row's first code byte
+  // row: LDS address of the row's first code byte.  RAW: a raw int8 code (the
+  // reference's bin_indices, any value), read signed: a negative one goes left
+  // at every split as the reference's signed `code <= bin` sends it (split
+  // bins are 0..126, or 255)
+  template <bool RAW>
   __device__ __forceinline__ void step(uint32_t row) {
     const uint32_t w = *(const lds_u32_t*)(uintptr_t)a;
-    const uint32_t c = *(const lds_u8_t*)(uintptr_t)(row + (w >> 16));
-    a = 2u * a + (c > (w & 0xffu) ? k1 : k0);
+    const uintptr_t at = row + (w >> 16);
+    const int c = RAW ? (int)*(const lds_i8_t*)at : (int)*(const lds_u8_t*)at;
+    a = 2u * a + (c > (int)(w & 0xffu) ? k1 : k0);
   }
 };
 
@@ -271,7 +269,7 @@ typedef __attribute__((address_space(3))) float lds_f32_t;
 // 4 (Hi + 1): every address is an add, and the trees' node words advance by
 // a uniform stride.  An idle walk (past n_trees, or row_on false) walks tree
 // 0 and stores nothing.
-template <int NW>
+template <int NW, bool RAW>
 __device__ __forceinline__ void walk_trees(int j_first, int n_trees, int G, bool row_on,
                                            uint32_t row_a, uint32_t nodes_a, uint32_t values_a,
                                            int Hi, int D, uint32_t out_a) {
@@ -290,7 +288,7 @@ __device__ __forceinline__ void walk_trees(int j_first, int n_trees, int G, bool
     }
     for (int d = 0; d < D; ++d) {
 #pragma unroll
-      for (int k = 0; k < NW; ++k) wk[k].step(row_a);
+      for (int k = 0; k < NW; ++k) wk[k].template step<RAW>(row_a);
     }
 #pragma unroll
     for (int k = 0; k < NW; ++k)
@@ -373,7 +371,7 @@ __global__ __launch_bounds__(kPredThreads) void predict_rows_kernel(
     // two in lock-step so that the LDS reads of one overlap those of the
     // other; max_depth steps on the complete tables (no leaf test)
     if (walker)
-      walk_trees<kPredWalks>(wt0, tc, G, wr < nr, lds_addr(rows_s + wr * Sp), lds_addr(nodes_s),
+      walk_trees<kPredWalks, false>(wt0, tc, G, wr < nr, lds_addr(rows_s + wr * Sp), lds_addr(nodes_s),
                              lds_addr(leaves_s), Hi, max_depth, lds_addr(vals_s + wr * (TC + 1)));
     __syncthreads();
     // ordered sums: trees t0 + j of class k are j = k, k + K, ... (t0 % K == 0)
@@ -410,13 +408,21 @@ __global__ __launch_bounds__(kPredThreads) void predict_rows_kernel(
 //   * wave 0 meanwhile adds the previous block's table to `out` in tree
 //     order (one lane per (row, class)), so the ordered sums run beside the
 //     walks; the value tables alternate between two buffers.
+// Bound by VALU work about as much as by the walks' LDS reads (four or seven
+// walks in lock-step are no faster than two), so a load's address is its place
+// in the block's run of bytes (no division by the row length, no row test: the
+// buffer's size ends the block), its place in LDS is found once, and raw codes
+// are compared as signed bytes instead of being mapped when stored.  100 trees of
+// depth 5, us before / now: 1M x 1000 raw codes 335 / 272; 300k rows of 1000, 696,
+// 400 raw codes 123 / 101, 100 / 90, 90 / 82, of 1000 and 500 native ones 97 /
+// 93, 82 / 76.
 // ---------------------------------------------------------------------------
 constexpr int kResThreads = 1024;
 constexpr int kResMaxQ = 4;  // 16-byte row loads per thread and block
 constexpr int kResWalks = 2;  // walks a walker thread advances in lock-step
 
 // RAW: the rows are raw int8 codes of stride S (a multiple of 8, read with
-// 8-byte loads, twice as many per thread) mapped by raw_walk_bytes, instead
+// 8-byte loads, twice as many per thread) and walked as signed bytes, instead
 // of native codes (S a multiple of 16) mapped by walk_bytes.
 template <bool RAW>
 __global__ __launch_bounds__(kResThreads) void predict_resident_kernel(
@@ -435,6 +441,7 @@ __global__ __launch_bounds__(kResThreads) void predict_resident_kernel(
   float* vals_s = reinterpret_cast<float*>(rows_s + RB * Sp);  // 2 x [RB][TV]
   const int tid = threadIdx.x;
   const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t bb = (uint32_t)num_bins * 0x01010101u;
   for (int i = tid; i < T * Hi; i += kResThreads) nodes_s[i] = cnode[i];
   for (int i = tid; i < T * L; i += kResThreads) leaves_s[i] = cleaf[i];
@@ -445,27 +452,35 @@ __global__ __launch_bounds__(kResThreads) void predict_resident_kernel(
   const int nq = RB * qpr;
   typedef uint32_t uq __attribute__((ext_vector_type(QW)));
   uq pre[NQ];
+  // a block's rows are one run of bytes (past the last row: zeros, no access);
+  // in LDS load q of row r moves by r pads
   auto prefetch = [&](int64_t b) {
+    const int64_t left = n - b * RB;
+    const __amdgpu_buffer_rsrc_t rs =
+        wgbm_rsrc(codes + b * RB * S, (uint32_t)((left < RB ? left : RB) * S));
 #pragma unroll
     for (int u = 0; u < NQ; ++u) {
-      const int q = u * kResThreads + tid;
-      const int r = q / qpr, c = q - r * qpr;
-      const int64_t row = b * RB + r;
-      pre[u] = uq{};
-      if (q < nq && row < n)
-        pre[u] = __builtin_nontemporal_load(reinterpret_cast<const uq*>(codes + row * S) + c);
+      const int at = (u * kResThreads + tid) * (4 * QW);
+      if (u * kResThreads + wave * 64 >= nq) break;  // uniform over the wave
+      if constexpr (RAW)
+        pre[u] = __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, kAuxStream);
+      else
+        pre[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, kAuxStream);
     }
   };
+  uint32_t to[NQ];  // the load's place in LDS
+#pragma unroll
+  for (int u = 0; u < NQ; ++u) {
+    const int q = u * kResThreads + tid;
+    to[u] = (uint32_t)(q * (4 * QW) + q / qpr * 4);
+  }
   auto stash = [&]() {
 #pragma unroll
     for (int u = 0; u < NQ; ++u) {
-      const int q = u * kResThreads + tid;
-      if (q < nq) {
-        const int r = q / qpr, c = q - r * qpr;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(rows_s + r * Sp + c * 4 * QW);
+      if (u * kResThreads + tid < nq) {
+        uint32_t* dst = reinterpret_cast<uint32_t*>(rows_s + to[u]);
 #pragma unroll
-        for (int k = 0; k < QW; ++k)
-          dst[k] = RAW ? raw_walk_bytes(pre[u][k]) : walk_bytes(pre[u][k], bb);
+        for (int k = 0; k < QW; ++k) dst[k] = RAW ? pre[u][k] : walk_bytes(pre[u][k], bb);
       }
     }
   };
@@ -514,8 +529,9 @@ __global__ __launch_bounds__(kResThreads) void predict_resident_kernel(
     } else if (walker) {
       const int64_t row0 = b * RB;
       const int nr = (int)(n - row0 < RB ? n - row0 : RB);
-      walk_trees<kResWalks>(wt0, T, G, wr < nr, lds_addr(rows_s + wr * Sp), lds_addr(nodes_s),
-                            lds_addr(leaves_s), Hi, max_depth, lds_addr(vt + wr * TV));
+      walk_trees<kResWalks, RAW>(wt0, T, G, wr < nr, lds_addr(rows_s + wr * Sp),
+                                 lds_addr(nodes_s), lds_addr(leaves_s), Hi, max_depth,
+                                 lds_addr(vt + wr * TV));
     }
     prev = b;
     __syncthreads();  // the walks are done: the row buffer can be refilled
@@ -550,6 +566,10 @@ int predict_resident_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int
   int64_t RB = (kBudget - 4 * T * H) / (Sp + 8 * (T + 1));
   RB = std::min<int64_t>(RB, (int64_t)kResMaxQ * kResThreads * 16 / S);
   RB = std::min<int64_t>(RB, 256);
+  // whole waves of rows: 65 rows are two passes of the sums' wave and walk
+  // groups that straddle waves (1M x 1000 raw codes, 65 / 64 rows a block: 334 / 287
+  // us; 300k x 400, 105 / 64 rows: 90 / 86; 300k x 200, 191 / 128 rows: 64 / 61)
+  if (RB > 64) RB -= RB % 64;
   if (RB < 8) return 0;
   *RB_out = (int32_t)RB;
   *lds_out = (size_t)(4 * T * H + RB * Sp + 8 * RB * (T + 1));
