@@ -536,8 +536,8 @@ int wgbm_predict_forest(const int8_t* bin_indices, int64_t n, int64_t n_feats,
   // Heap path, for enough trees and rows: the flat tables become heap tables
   // of depth D = floor(log2(max_nodes)) - 1 (flatten_tree's max_nodes =
   // 2^(max_depth+1)), walked by the LDS predictors.  Rows of a multiple of 8
-  // bytes are read as they are by the resident predictor (a negative code
-  // read as 0, which every split sends left); otherwise the codes get a
+  // bytes are read as they are by the resident predictor (compared as signed
+  // bytes: every split sends a negative code left); otherwise the codes get a
   // native copy (num_bins 127: a negative code becomes the byte 127, which
   // every split sends left; 127 becomes 128, which every split bin <= 126
   // sends right; the other codes stay).  A
