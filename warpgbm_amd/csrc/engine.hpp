@@ -223,14 +223,14 @@ struct LevelNext {
   // node_scan_kernel: the next level's live-era masks (des_alive_kernel's
   // output for the children, [2 * T * nodes][ceil(E / 32)]), or null
   uint32_t* alive_next;
-  float mcw;
+  float mcw;  // of the masks and of level_scan_kernel<true>'s plan: live segments
 };
+template <bool LIVE>
 __global__ void level_scan_kernel(int32_t nb, PartSums ps, int32_t T, int32_t nodes, int32_t E,
                                   int64_t n_pos, const int64_t* seg, const int32_t* present,
                                   const int32_t* split_l, LevelNext nx, int32_t n_list,
                                   int32_t tile_rows, int32_t max_tiles, Tile* tiles,
-                                  int32_t* key_tile_start, int32_t* n_tiles,
-                                  int32_t plan_present, float mcw);
+                                  int32_t* key_tile_start, int32_t* n_tiles);
 // One-era split levels in one pass: route, rank and place every position
 // (route_kernel + scatter_kernel without the block prefix between them), for
 // levels of at most kPartition1MaxNodes (tree, node)s.

@@ -823,9 +823,9 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
           r = era_tile_plan(e, nc, (n_tn + nc - 1) / nc, &lp);
           if (r) return r;
           if (!planned) {  // (else by the previous level's scan)
-            hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
-                               (int64_t)0, lp.n_list, (const int32_t*)nullptr, (int32_t)lp.R, 0,
-                               (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
+            hipLaunchKernelGGL(plan_tiles_kernel<true>, dim3(1), dim3(1024), 0, st,
+                               e->seg[cur] + k0, (int64_t)0, lp.n_list, (const int32_t*)nullptr,
+                               (int32_t)lp.R, 0, (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
                                e->present[cur] + c0, E, mcw);
             WGBM_LAUNCH_CHECK();
           }
@@ -928,7 +928,7 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
               if (ra2) return ra2;
               e->root_tiles_cap = max_tiles;
             }
-            hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur],
+            hipLaunchKernelGGL(plan_tiles_kernel<false>, dim3(1), dim3(1024), 0, st, e->seg[cur],
                                (int64_t)0, n_list, list, (int32_t)R, 0, (int32_t)max_tiles,
                                e->root_tiles, e->root_kts, e->root_hn, (const int32_t*)nullptr, 1,
                                0.0f);
@@ -939,7 +939,7 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
           kts_d = e->root_kts;
           hn_d = e->root_hn;
         } else if (!(subtract && planned)) {
-          hipLaunchKernelGGL(plan_tiles_kernel, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
+          hipLaunchKernelGGL(plan_tiles_kernel<false>, dim3(1), dim3(1024), 0, st, e->seg[cur] + k0,
                              (int64_t)0, n_list, list, (int32_t)R, 0, (int32_t)max_tiles,
                              e->htiles, e->hkts, e->hn, (const int32_t*)nullptr, 1, 0.0f);
           WGBM_LAUNCH_CHECK();
@@ -1125,11 +1125,11 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
           const int r = era_tile_plan(e, 2 * (int64_t)n_tn, 1, &lp);
           if (r) return r;
         }
-        hipLaunchKernelGGL(level_scan_kernel, dim3(1), dim3(1024), 0, st, (int32_t)e->nb, e->ps,
-                           T, nodes, E, n_pos, e->seg[cur], e->present[cur], e->split_l, nx,
+        hipLaunchKernelGGL((next_tiles ? level_scan_kernel<true> : level_scan_kernel<false>),
+                           dim3(1), dim3(1024), 0, st, (int32_t)e->nb, e->ps, T, nodes, E, n_pos,
+                           e->seg[cur], e->present[cur], e->split_l, nx,
                            next_hist || next_tiles ? lp.n_list : 0, (int32_t)lp.R,
-                           (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn,
-                           next_tiles ? 1 : 0, mcw);
+                           (int32_t)lp.max_tiles, e->htiles, e->hkts, e->hn);
         WGBM_LAUNCH_CHECK();
         planned = next_hist || next_tiles;
       } else {

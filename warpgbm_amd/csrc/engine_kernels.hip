@@ -1670,12 +1670,13 @@ __global__ __launch_bounds__(256) void leaf_rows_kernel(const int32_t* __restric
 // first n_list entries of key_list_next; skipped when n_list is 0).  The
 // prefix and the node scan's outputs are read back by the same workgroup
 // after a barrier.
+template <bool LIVE>
 __global__ __launch_bounds__(1024) void level_scan_kernel(
     int32_t nb, PartSums ps, int32_t T, int32_t nodes, int32_t E, int64_t n_pos,
     const int64_t* __restrict__ seg, const int32_t* __restrict__ present,
     const int32_t* __restrict__ split_l, LevelNext nx, int32_t n_list, int32_t tile_rows,
     int32_t max_tiles, Tile* __restrict__ tiles, int32_t* __restrict__ key_tile_start,
-    int32_t* __restrict__ n_tiles, int32_t plan_present, float mcw) {
+    int32_t* __restrict__ n_tiles) {
   block_scan_body(nb, ps);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1734,12 +1735,19 @@ __global__ __launch_bounds__(1024) void level_scan_kernel(
   }
   if (n_list <= 0) return;  // uniform
   __syncthreads();
-  // plan_present: the tiles of every live segment of the next level (the era
-  // levels of few large segments), else those of its key list
-  plan_tiles_body(nx.seg_next, 0, n_list, plan_present ? nullptr : nx.key_list_next, tile_rows, 0,
-                  max_tiles, tiles, key_tile_start, n_tiles,
-                  plan_present ? nx.present_next : nullptr, E, mcw);
+  // LIVE: the tiles of every live segment of the next level (the era levels of
+  // few large segments), else those of its key list
+  plan_tiles_body<LIVE>(nx.seg_next, 0, n_list, LIVE ? nullptr : nx.key_list_next, tile_rows, 0,
+                        max_tiles, tiles, key_tile_start, n_tiles, nx.present_next, E, nx.mcw);
 }
+template __global__ void level_scan_kernel<false>(int32_t, PartSums, int32_t, int32_t, int32_t,
+                                                  int64_t, const int64_t*, const int32_t*,
+                                                  const int32_t*, LevelNext, int32_t, int32_t,
+                                                  int32_t, Tile*, int32_t*, int32_t*);
+template __global__ void level_scan_kernel<true>(int32_t, PartSums, int32_t, int32_t, int32_t,
+                                                 int64_t, const int64_t*, const int32_t*,
+                                                 const int32_t*, LevelNext, int32_t, int32_t,
+                                                 int32_t, Tile*, int32_t*, int32_t*);
 
 // One-era split search fused with the leaf / record step: one lane per
 // (node, local feature) scans the node's histogram as split_level_e1_kernel
@@ -2043,8 +2051,8 @@ __global__ __launch_bounds__(1024) void level_scan_e1_kernel(
   if (!plan) return;  // uniform
   if (n_tn > 1024) {
     __syncthreads();
-    plan_tiles_body(nx.seg_next, 0, 2 * n_tn, nx.key_list_next, tile_rows, 0, max_tiles, tiles,
-                    key_tile_start, n_tiles);
+    plan_tiles_body<false>(nx.seg_next, 0, 2 * n_tn, nx.key_list_next, tile_rows, 0, max_tiles,
+                           tiles, key_tile_start, n_tiles);
     return;
   }
   // tiles per entry (plan_tiles_body's count, rounding up); key c0 spans

@@ -1001,8 +1001,8 @@ __global__ __launch_bounds__(1024) void hist_prep_kernel(
     int32_t* __restrict__ n_tiles, FeatMapArgs fm, uint32_t* __restrict__ key_max) {
   if ((int)blockIdx.x >= n_part) {
     if (plan && (int)blockIdx.x == n_part)
-      plan_tiles_body(seg, n, n_keys, nullptr, tile_rows, 1, max_tiles, tiles, key_tile_start,
-                      n_tiles);
+      plan_tiles_body<false>(seg, n, n_keys, nullptr, tile_rows, 1, max_tiles, tiles,
+                             key_tile_start, n_tiles);
     else if (fm.feat_idx)
       feature_map_body(fm);
     return;
@@ -1079,16 +1079,22 @@ __global__ __launch_bounds__(256) void hist_key_max_kernel(
   if (threadIdx.x == 0 && m) atomicMax(key_max + tl.key, m);
 }
 
+template <bool LIVE>
 __global__ __launch_bounds__(1024) void plan_tiles_kernel(
     const int64_t* __restrict__ seg, int64_t total_rows, int32_t n_keys,
     const int32_t* __restrict__ key_list, int32_t tile_rows, int32_t nearest,
     int32_t max_tiles, Tile* __restrict__ tiles, int32_t* __restrict__ key_tile_start,
     int32_t* __restrict__ n_tiles, const int32_t* __restrict__ present, int32_t num_eras,
     float mcw) {
-  plan_tiles_body(seg, total_rows, n_keys, key_list, tile_rows, nearest, max_tiles, tiles,
-                  key_tile_start, n_tiles, present, num_eras, mcw);
+  plan_tiles_body<LIVE>(seg, total_rows, n_keys, key_list, tile_rows, nearest, max_tiles, tiles,
+                        key_tile_start, n_tiles, present, num_eras, mcw);
 }
-
+template __global__ void plan_tiles_kernel<false>(const int64_t*, int64_t, int32_t, const int32_t*,
+                                                  int32_t, int32_t, int32_t, Tile*, int32_t*,
+                                                  int32_t*, const int32_t*, int32_t, float);
+template __global__ void plan_tiles_kernel<true>(const int64_t*, int64_t, int32_t, const int32_t*,
+                                                 int32_t, int32_t, int32_t, Tile*, int32_t*,
+                                                 int32_t*, const int32_t*, int32_t, float);
 
 // --------------------------------------------------------------------------
 // era regrouping for the ABI path: row list -> era-grouped positions.

@@ -15,10 +15,12 @@ namespace wgbm {
 // a small remainder, so the workgroups of a launch carry even work.  keys:
 // either all n_keys (list == nullptr) or the first *n_list entries of
 // key_list.  seg: int64 [n_keys+1] (nullptr => a single segment [0, total)).
-// With present (and no list), keys of an absent node (key / num_eras) and
-// dead segments (des_segment_dead) get no tiles.
+// LIVE (no list): keys of an absent node (present[key / num_eras] == 0) and
+// dead segments (des_segment_dead) get no tiles; without it those arguments
+// are not read, nor compiled into the other planners.
 // --------------------------------------------------------------------------
 // (blockDim.x == 1024)
+template <bool LIVE>
 __device__ inline void plan_tiles_body(
     const int64_t* __restrict__ seg, int64_t total_rows, int32_t n_keys,
     const int32_t* __restrict__ key_list, int32_t tile_rows, int32_t nearest,
@@ -32,7 +34,9 @@ __device__ inline void plan_tiles_body(
     key = key_list ? key_list[i] : i;
     b0 = (key >= 0 && seg) ? seg[key] : 0;
     b1 = key < 0 ? 0 : (seg ? seg[key + 1] : total_rows);
-    if (present && (!present[key / num_eras] || des_segment_dead(b1 - b0, mcw))) key = -1;
+    if constexpr (LIVE) {
+      if (!present[key / num_eras] || des_segment_dead(b1 - b0, mcw)) key = -1;
+    }
   };
   // segment lengths are below 2^31 (positions are int32): 32-bit divisions
   auto count = [&](int64_t len64) -> int64_t {
