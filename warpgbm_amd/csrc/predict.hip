@@ -496,6 +496,9 @@ __global__ __launch_bounds__(kResThreads) void predict_resident_kernel(
       float a = *o;
       // tree order; eight loads issued ahead of their sequential adds
       int j = k;
+      // (one wave runs this loop, bound by its instruction fetch: starting at
+      // 28 of 32 bytes it took 4% more of a call of 16 classes than at 4 .. 16)
+      __asm__ volatile(".p2align 6");
       for (; j + 7 * K < T; j += 8 * K) {
         float x[8];
 #pragma unroll
