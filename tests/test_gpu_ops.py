@@ -431,6 +431,9 @@ RESIDENT_CASES = [
     (True, 4096, 8, 1, 30, 5), (True, 4097, 520, 1, 60, 5), (True, 20_001, 1000, 1, 100, 5),
     (True, 16_449, 1504, 1, 40, 4), (False, 63, 520, 1, 60, 5), (False, 129, 600, 3, 30, 5),
     (False, 16_385, 1000, 1, 100, 5), (False, 20_003, 640, 10, 12, 4),
+    # blocks of 122 rows, which cover these rows with one on each CU (64 do not),
+    # and one row past them
+    (True, 31_232, 536, 1, 40, 4), (True, 31_233, 536, 1, 40, 4),
 ]
 
 

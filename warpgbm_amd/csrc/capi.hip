@@ -406,7 +406,7 @@ static int predict_heap_impl(const int8_t* codes, int64_t n, int64_t codes_strid
   int dev = 0, n_cu = 0;
   WGBM_CHECK(hipGetDevice(&dev));
   WGBM_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-  const bool resident = predict_resident_plan(codes_stride, K, H, n_rounds, &RB, &lds) != 0;
+  const bool resident = predict_resident_plan(n, codes_stride, K, H, n_rounds, &RB, &lds) != 0;
   // The column-block predictor where two of its workgroups share a CU, or
   // nothing else keeps the trees in LDS.  1M x 100, 32 bins, us with the row
   // walkers / with it: 2000 trees of depth 6, 10 classes 3600 / 1910; 100 trees,
@@ -498,7 +498,7 @@ static int predict_forest_raw(const int8_t* raw, int64_t n, int64_t n_feats,
   int32_t RB = 0;
   size_t lds = 0;
   if (n_feats % 8 != 0 || ((uintptr_t)raw % 8) != 0 ||
-      !predict_resident_plan(n_feats, 1, H, n_trees, &RB, &lds, true))
+      !predict_resident_plan(n, n_feats, 1, H, n_trees, &RB, &lds, true))
     return -1;
   int dev = 0, n_cu = 0;
   WGBM_CHECK(hipGetDevice(&dev));

@@ -558,8 +558,8 @@ template __global__ void predict_resident_kernel<true>(const int8_t*, int64_t, i
 
 // block shape of predict_resident_kernel: 0 when the trees do not fit (raw:
 // rows of raw codes, S a multiple of 8; else native rows, S a multiple of 16)
-int predict_resident_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int32_t* RB_out,
-                          size_t* lds_out, bool raw) {
+int predict_resident_plan(int64_t n, int64_t S, int32_t K, int32_t H, int32_t n_rounds,
+                          int32_t* RB_out, size_t* lds_out, bool raw) {
   constexpr int64_t kBudget = 150 * 1024;
   const int64_t T = (int64_t)n_rounds * K;
   // complete tables: (H - 1) / 2 node words and (H + 1) / 2 values per tree
@@ -571,8 +571,11 @@ int predict_resident_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int
   RB = std::min<int64_t>(RB, 256);
   // whole waves of rows: 65 rows are two passes of the sums' wave and walk
   // groups that straddle waves (1M x 1000 raw codes, 65 / 64 rows a block: 334 / 287
-  // us; 300k x 400, 105 / 64 rows: 90 / 86; 300k x 200, 191 / 128 rows: 64 / 61)
-  if (RB > 64) RB -= RB % 64;
+  // us; 300k x 400, 105 / 64 rows: 90 / 86; 300k x 200, 191 / 128 rows: 64 / 61),
+  // unless only the larger blocks cover the rows with one on each CU (60k x
+  // 250, 40 trees of depth 5, 8 classes, 244 / 192 rows: 25 / 30)
+  const int64_t whole = RB - RB % 64;
+  if (RB > 64 && !(n <= 256 * RB && n > 256 * whole)) RB = whole;
   if (RB < 8) return 0;
   *RB_out = (int32_t)RB;
   *lds_out = (size_t)(4 * T * H + RB * Sp + 8 * RB * (T + 1));
