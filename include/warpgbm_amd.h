@@ -205,6 +205,14 @@ int wgbm_predict_heap(const int8_t* codes, int64_t n, int64_t codes_stride, int3
                       int32_t n_rounds, int32_t K, int32_t H, int32_t max_depth,
                       float learning_rate, float* out, void* stream);
 
+/* The kernel a wgbm_predict_heap call of these sizes takes (codes on 16
+ * bytes): 0 = a thread per (row, class) over the heap tables, 1 = row blocks,
+ * trees in chunks, 2 = row blocks, all trees resident in LDS, 3 = column
+ * blocks; -1 for sizes out of range.  Every kernel gives the same result.  No
+ * device call is made. */
+int wgbm_predict_heap_path(int64_t n, int64_t codes_stride, int32_t n_rounds, int32_t K,
+                           int32_t max_depth);
+
 /* In-place row softmax of float32 [n, K] (warpgbm/metrics.py:12-15). */
 int wgbm_softmax_rows(float* x, int64_t n, int32_t K, void* stream);
 

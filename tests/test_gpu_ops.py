@@ -388,18 +388,30 @@ def _random_heap(rng, R, K, depth, F, B):
     return feat, binv, leaf, tables
 
 
-# name, rows, features, bins, classes, rounds, depth: the LDS-resident
+HEAP, ROWS, RESIDENT, COLS = range(4)  # wgbm_predict_heap_path
+
+
+def heap_path(N, F, K, R, depth):
+    return _lib.load().wgbm_predict_heap_path(N, D.codes_stride(F), R, K, depth)
+
+
+# name, kernel, rows, features, bins, classes, rounds, depth: the LDS-resident
 # predictor (also with single-leaf trees and blocks of 9 rows), the row-block
-# predictor (partial last tree chunk and row block, deep trees, one round
-# per tree chunk) and the heap walker
+# predictor (partial last tree chunk and row block, rows wider than 511 bytes,
+# many classes, deep trees, one round per tree chunk), the column blocks with a
+# partial chunk and the heap walker
 PRED_CASES = [
-    ("resident", 5000, 40, 16, 1, 30, 5),
-    ("rows_partial_chunk", 7001, 100, 32, 10, 23, 6),
-    ("rows_deep", 3000, 20, 8, 1, 50, 9),
-    ("rows_one_round_per_chunk", 2000, 30, 8, 3, 4, 10),
-    ("resident_depth0", 500, 10, 4, 10, 200, 0),
-    ("heap", 3000, 30, 8, 10, 3, 10),
-    ("heap_depth0", 500, 10, 4, 10, 2000, 0),
+    ("resident", RESIDENT, 5000, 600, 16, 1, 30, 5),
+    ("resident_narrow", RESIDENT, 500, 40, 16, 10, 60, 2),
+    ("cols", COLS, 5000, 40, 16, 1, 30, 5),
+    ("rows_partial_chunk", ROWS, 7001, 600, 32, 10, 23, 6),
+    ("cols_partial_chunk", COLS, 7001, 100, 32, 10, 23, 6),
+    ("rows_deep", ROWS, 3000, 20, 8, 1, 50, 9),
+    ("rows_one_round_per_chunk", ROWS, 2000, 30, 8, 3, 4, 10),
+    ("resident_depth0", RESIDENT, 500, 10, 4, 10, 200, 0),
+    ("rows_shallow_many_trees", ROWS, 3000, 40, 16, 10, 120, 4),
+    ("heap", HEAP, 3000, 30, 8, 10, 3, 10),
+    ("heap_depth0", HEAP, 500, 10, 4, 10, 2000, 0),
 ]
 
 
@@ -407,10 +419,11 @@ PRED_CASES = [
 def test_predict_heap_paths_bit_exact(gpu, case):
     """wgbm_predict_heap (the estimator's predictor) on raw codes with values
     outside [0, B) equals the reference-table walk (warpgbm/cuda/predict.cu:
-    23-44, trees added in (round, class) order) bit for bit, whichever of its
-    three kernels the shape selects."""
-    name, N, F, B, K, R, depth = case
+    23-44, trees added in (round, class) order) bit for bit, by each of its
+    four kernels."""
+    name, path, N, F, B, K, R, depth = case
     print_case("predict_heap", name)
+    assert heap_path(N, F, K, R, depth) == path
     rng = np.random.default_rng(zlib.crc32(name.encode()))
     raw = rng.integers(-2, B + 3, (N, F)).astype(np.int8)
     feat, binv, leaf, tables = _random_heap(rng, R, K, depth, F, B)
@@ -454,6 +467,7 @@ def test_predict_resident_row_blocks_bit_exact(gpu, case):
         padded = np.pad(tables, ((0, 0), (0, 1), (0, 0)))  # 2^(depth + 1) slots
         node_kernel.predict_forest(t(raw), t(padded), 0.1, out.reshape(-1))
     else:
+        assert heap_path(N, F, K, R, depth) == RESIDENT
         codes = D.codes_from_int8(D.upload_int8(raw, dev), False, 32)[0]
         D.predict_heap(codes, t(feat), t(binv), t(leaf), R, K, depth, 0.1, out)
     ref = clib.predict_tables(raw, tables, F32(0.1), out0, np.tile(np.arange(K, dtype=np.int32), R))
@@ -463,11 +477,12 @@ def test_predict_resident_row_blocks_bit_exact(gpu, case):
 # rows, features, bins, classes, rounds, depth: the column-block predictor's row
 # blocks (256) and stride groups (16 columns), values through LDS (below 8
 # classes) or sums in registers (one or two classes a wave, to 32), the extension
-# of trees shallower than 4, bins up to the largest, partial chunks
+# of trees shallower than 4, bins up to the largest, partial chunks, more than
+# one block a CU
 COLS_CASES = [
     (1, 1, 2, 1, 3, 1), (255, 16, 127, 1, 40, 4), (257, 17, 32, 7, 9, 3), (700, 33, 10, 8, 30, 6),
-    (1025, 300, 32, 17, 5, 5), (513, 120, 127, 32, 4, 2), (300, 380, 63, 3, 12, 8),
-    (300, 50, 16, 33, 3, 5), (300, 505, 16, 9, 3, 6),
+    (1025, 300, 32, 17, 40, 6), (513, 120, 127, 32, 4, 2), (300, 380, 63, 3, 12, 8),
+    (66_000, 20, 32, 7, 10, 4), (300, 50, 16, 33, 3, 5), (300, 505, 16, 9, 3, 6),
 ]
 
 
@@ -478,6 +493,7 @@ def test_predict_heap_column_blocks_bit_exact(gpu, case):
     included, and one case past each of its limits."""
     N, F, B, K, R, depth = case
     print_case("predict_heap column blocks", case)
+    assert (heap_path(N, F, K, R, depth) == COLS) == (K <= 32 and F <= 384)
     rng = np.random.default_rng(N + F)
     raw = rng.integers(-2, min(B + 3, 128), (N, F)).astype(np.int8)
     feat, binv, leaf, tables = _random_heap(rng, R, K, depth, F, B)

@@ -401,25 +401,15 @@ static int predict_heap_impl(const int8_t* codes, int64_t n, int64_t codes_strid
   if (n == 0) return 0;
   WGBM_REQUIRE(codes && out && (n_rounds == 0 || (feat && bin && leaf)), "null pointer");
   if (n_rounds == 0) return 0;
-  int32_t RB = 0, TC = 0;
-  size_t lds = 0;
   int dev = 0, n_cu = 0;
   WGBM_CHECK(hipGetDevice(&dev));
   WGBM_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-  const bool resident = predict_resident_plan(n, codes_stride, K, H, n_rounds, &RB, &lds) != 0;
-  // The column-block predictor where two of its workgroups share a CU, or
-  // nothing else keeps the trees in LDS.  1M x 100, 32 bins, us with the row
-  // walkers / with it: 2000 trees of depth 6, 10 classes 3600 / 1910; 100 trees,
-  // one class: depth 6 239 / 169, depth 5 213 / 136, depth 3 161 / 128; 200k x
-  // 300, 3 classes, 300 trees of depth 8 430 / 243; but one workgroup a CU,
-  // 200k x 300, 100 trees of depth 5: 64 / 81.
-  int32_t DX = 0, waves = 0, cols_tc = 0;
-  bool vt = false;
-  size_t cols_lds = 0;
-  if (predict_cols_plan(codes_stride, K, max_depth, n_rounds, &DX, &waves, &cols_tc, &vt,
-                        &cols_lds) &&
-      (uintptr_t)codes % 16 == 0 && (!resident || cols_lds <= 80 * 1024)) {
-    const int64_t T = (int64_t)n_rounds * K, words = kColsUni + (int64_t(2) << DX) - (1 << kColsTop);
+  const PredictPlan pl =
+      predict_plan(n, codes_stride, (uintptr_t)codes % 16 == 0, K, max_depth, n_rounds);
+  if (pl.kind == kPredictCols) {
+    const int32_t DX = pl.DX;
+    const int64_t T = (int64_t)n_rounds * K;
+    const int64_t words = kColsUni + (int64_t(2) << DX) - (1 << kColsTop);
     uint32_t* uni = (uint32_t*)scratch_get(S(stream), sizeof(uint32_t) * (size_t)(T * words), 13);
     WGBM_REQUIRE(uni, "scratch allocation failed");
     uint32_t* tab = uni + T * kColsUni;
@@ -434,14 +424,14 @@ static int predict_heap_impl(const int8_t* codes, int64_t n, int64_t codes_strid
                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       attr_c = true;
     }
-    hipLaunchKernelGGL((vt ? predict_cols_kernel<true> : predict_cols_kernel<false>),
-                       dim3(nblocks(n, kColsRows)), dim3(64 * waves), cols_lds, S(stream), codes,
+    hipLaunchKernelGGL((pl.vt ? predict_cols_kernel<true> : predict_cols_kernel<false>),
+                       dim3(nblocks(n, kColsRows)), dim3(64 * pl.waves), pl.lds, S(stream), codes,
                        n, codes_stride, num_bins, (const uint32_t*)uni, (const uint32_t*)tab,
-                       (int32_t)T, K, DX, cols_tc, out, skip);
+                       (int32_t)T, K, DX, pl.TC, out, skip);
     WGBM_LAUNCH_CHECK();
     return 0;
   }
-  const bool rows = !resident && predict_rows_plan(codes_stride, K, H, n_rounds, &RB, &TC, &lds);
+  const bool resident = pl.kind == kPredictResident, rows = pl.kind == kPredictRows;
   uint32_t* cnode = nullptr;
   float* cleaf = nullptr;
   if (resident || rows) {
@@ -464,10 +454,10 @@ static int predict_heap_impl(const int8_t* codes, int64_t n, int64_t codes_strid
       attr_r = true;
     }
     // one persistent workgroup per CU (fewer when there are fewer blocks)
-    const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(n_cu, nblocks(n, RB)));
-    hipLaunchKernelGGL(predict_resident_kernel<false>, dim3((unsigned)grid), dim3(1024), lds,
+    const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(n_cu, nblocks(n, pl.RB)));
+    hipLaunchKernelGGL(predict_resident_kernel<false>, dim3((unsigned)grid), dim3(1024), pl.lds,
                        S(stream), codes, n, codes_stride, num_bins, (const uint32_t*)cnode,
-                       (const float*)cleaf, n_rounds * K, K, max_depth, RB, out, skip);
+                       (const float*)cleaf, n_rounds * K, K, max_depth, pl.RB, out, skip);
   } else if (rows) {
     static bool attr = false;
     if (!attr) {
@@ -475,9 +465,9 @@ static int predict_heap_impl(const int8_t* codes, int64_t n, int64_t codes_strid
                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       attr = true;
     }
-    hipLaunchKernelGGL(predict_rows_kernel, dim3(nblocks(n, RB)), dim3(1024), lds, S(stream),
+    hipLaunchKernelGGL(predict_rows_kernel, dim3(nblocks(n, pl.RB)), dim3(1024), pl.lds, S(stream),
                        codes, n, codes_stride, num_bins, (const uint32_t*)cnode,
-                       (const float*)cleaf, n_rounds, K, max_depth, RB, TC, out, skip);
+                       (const float*)cleaf, n_rounds, K, max_depth, pl.RB, pl.TC, out, skip);
   } else {
     hipLaunchKernelGGL(predict_heap_kernel, dim3(nblocks(n * K, 256)), dim3(256), 0, S(stream),
                        codes, n, codes_stride, num_bins, feat, bin, leaf, n_rounds, K, H,
@@ -525,6 +515,13 @@ static int predict_forest_raw(const int8_t* raw, int64_t n, int64_t n_feats,
 }
 
 extern "C" {
+
+int wgbm_predict_heap_path(int64_t n, int64_t codes_stride, int32_t n_rounds, int32_t K,
+                           int32_t max_depth) {
+  if (n < 0 || codes_stride < 1 || n_rounds < 1 || K < 1 || max_depth < 0 || max_depth > 29)
+    return -1;
+  return predict_plan(n, codes_stride, true, K, max_depth, n_rounds).kind;
+}
 
 int wgbm_predict_forest(const int8_t* bin_indices, int64_t n, int64_t n_feats,
                         const float* tree_tensor, int64_t n_trees, int64_t max_nodes,

@@ -472,14 +472,10 @@ __global__ void predict_cols_kernel(const int8_t* codes, int64_t n, int64_t S, i
                                     const uint32_t* uni, const uint32_t* tab, int32_t T,
                                     int32_t K, int32_t DX, int32_t TC, float* out,
                                     const int32_t* skip);
-int predict_cols_plan(int64_t S, int32_t K, int32_t D, int32_t n_rounds, int32_t* DX_out,
-                      int32_t* waves_out, int32_t* TC_out, bool* vt_out, size_t* lds_out);
 __global__ void predict_rows_kernel(const int8_t* codes, int64_t n, int64_t S, int32_t num_bins,
                                     const uint32_t* cnode, const float* cleaf, int32_t n_rounds,
                                     int32_t K, int32_t max_depth, int32_t RB, int32_t TC,
                                     float* out, const int32_t* skip);
-int predict_rows_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int32_t* RB_out,
-                      int32_t* TC_out, size_t* lds_out);
 template <bool RAW>
 __global__ void predict_resident_kernel(const int8_t* codes, int64_t n, int64_t S,
                                         int32_t num_bins, const uint32_t* cnode,
@@ -488,6 +484,17 @@ __global__ void predict_resident_kernel(const int8_t* codes, int64_t n, int64_t 
                                         const int32_t* skip);
 int predict_resident_plan(int64_t n, int64_t S, int32_t K, int32_t H, int32_t n_rounds,
                           int32_t* RB_out, size_t* lds_out, bool raw = false);
+// kernel and block shape of a wgbm_predict_heap call (codes on 16 bytes or not)
+enum { kPredictHeap = 0, kPredictRows = 1, kPredictResident = 2, kPredictCols = 3 };
+struct PredictPlan {
+  int32_t kind = kPredictHeap;
+  int32_t RB = 0, TC = 0;     // rows a block, trees a chunk
+  int32_t DX = 0, waves = 0;  // column blocks: depth of the tables, waves
+  bool vt = false;            // column blocks: values through LDS
+  size_t lds = 0;
+};
+PredictPlan predict_plan(int64_t n, int64_t S, bool aligned16, int32_t K, int32_t D,
+                         int32_t n_rounds);
 __global__ void softmax_rows_kernel(float* x, int64_t n, int32_t K);
 __global__ void importance_add_kernel(float* acc, int32_t F, int32_t E, const float* gain,
                                       const int64_t* node, const int64_t* fstart);

@@ -371,8 +371,9 @@ __global__ __launch_bounds__(kPredThreads) void predict_rows_kernel(
     // two in lock-step so that the LDS reads of one overlap those of the
     // other; max_depth steps on the complete tables (no leaf test)
     if (walker)
-      walk_trees<kPredWalks, false>(wt0, tc, G, wr < nr, lds_addr(rows_s + wr * Sp), lds_addr(nodes_s),
-                             lds_addr(leaves_s), Hi, max_depth, lds_addr(vals_s + wr * (TC + 1)));
+      walk_trees<kPredWalks, false>(wt0, tc, G, wr < nr, lds_addr(rows_s + wr * Sp),
+                                    lds_addr(nodes_s), lds_addr(leaves_s), Hi, max_depth,
+                                    lds_addr(vals_s + wr * (TC + 1)));
     __syncthreads();
     // ordered sums: trees t0 + j of class k are j = k, k + K, ... (t0 % K == 0)
 #pragma unroll
@@ -584,7 +585,7 @@ int predict_resident_plan(int64_t n, int64_t S, int32_t K, int32_t H, int32_t n_
 
 // block shape of predict_rows_kernel: 0 when the trees or rows do not fit
 // (then predict_heap_kernel is used)
-int predict_rows_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int32_t* RB_out,
+static int predict_rows_plan(int64_t S, int32_t K, int32_t H, int32_t n_rounds, int32_t* RB_out,
                       int32_t* TC_out, size_t* lds_out) {
   constexpr int64_t kBudget = 64 * 1024;
   // complete tables: (H - 1) / 2 node words and (H + 1) / 2 values per tree
@@ -850,7 +851,7 @@ template __global__ void predict_cols_kernel<true>(const int8_t*, int64_t, int64
 
 // block shape of predict_cols_kernel: waves, trees per chunk, whether values go
 // through LDS; 0 when a chunk of one round does not fit
-int predict_cols_plan(int64_t S, int32_t K, int32_t D, int32_t n_rounds, int32_t* DX_out,
+static int predict_cols_plan(int64_t S, int32_t K, int32_t D, int32_t n_rounds, int32_t* DX_out,
                       int32_t* waves_out, int32_t* TC_out, bool* vt_out, size_t* lds_out) {
   const int32_t DX = std::max(D, kColsTop);
   if (S % 16 != 0 || DX > 8 || S > 511) return 0;
@@ -876,6 +877,106 @@ int predict_cols_plan(int64_t S, int32_t K, int32_t D, int32_t n_rounds, int32_t
   *vt_out = vt;
   *lds_out = (size_t)lds;
   return 1;
+}
+
+// ---------------------------------------------------------------------------
+// Which kernel a call of wgbm_predict_heap takes.
+// ---------------------------------------------------------------------------
+// More rows than one block of the column-block predictor on every CU, and two of
+// its workgroups on a CU: it is taken.  1M x 100, 32 bins, us with the row
+// walkers / with it: 2000 trees of depth 6, 10 classes 3600 / 1910; 100 trees, one
+// class: depth 6 239 / 169, depth 5 213 / 136, depth 3 161 / 128; 200k x 300, 3
+// classes, 300 trees of depth 8 430 / 243.
+//
+// Otherwise its time is that of one block, whatever the row count (or of as many
+// as a CU gets): a class's trees one after the other, or a sixteenth of all
+// trees.  The other kernels cut their row blocks smaller the more trees there are
+// and fill the CUs (500 rows, 1700 trees of depth 1, 17 classes: 14 us against
+// 118; 912 rows, 47 trees of depth 1: 14 / 11; 200k x 300, 100 trees of depth 5:
+// 64 / 81), but lose to it where trees are few for the rows or deep (4000 rows,
+// 120 trees of depth 8, 3 classes: 61 / 36).  So the times of both are estimated
+// and the smaller is taken.  The estimates (us) were fitted to 7920 measured
+// shapes (300 .. 300k rows, rows of 32 .. 384 bytes, 1 .. 32 classes, depths 0 ..
+// 8, 2 .. 200 rounds): half of them within 5%, nine of ten within 16%; the
+// kernel taken is on average 0.3% slower than the better of the two, less than
+// 10% in 99 of 100 shapes.  Always taking it lost 5% or more in a quarter of them.
+struct PredictSizes {
+  int64_t n, S, K, R, T, H;
+  int D;
+  int64_t RB, TC;
+};
+static double ceil_div(int64_t a, int64_t b) { return (double)((a + b - 1) / b); }
+// blocks of rows that a CU gets, one after the other
+static double blocks_per_cu(int64_t n, int64_t rows) {
+  return ceil_div((n + rows - 1) / rows, 256);
+}
+// rows of a wave that start on one LDS bank, but for the first
+static double lds_conflicts(int64_t stride) {
+  int64_t g = 64;
+  while (stride % g) g /= 2;
+  return (double)(g - 1);
+}
+
+static double est_cols(const PredictSizes& p, const PredictPlan& c) {
+  const double below = c.DX - kColsTop;  // levels walked row by row
+  const int64_t GW = (int64_t(2) << c.DX) - (1 << kColsTop);
+  const double chunks = ceil_div(p.T, c.TC), blocks = blocks_per_cu(p.n, kColsRows);
+  if (c.vt)
+    return 5.1 + blocks * (ceil_div(p.T, 16) * (0.55 + 0.283 * below) +
+                           0.030 * p.R * ceil_div(p.K, 4) + 1.18 * chunks + 0.0101 * p.S);
+  return 7.0 + blocks * (p.R * ceil_div(p.K, c.waves) * (0.317 + 0.155 * below + 0.0281 * c.waves) +
+                         chunks * (0.316 + 0.12 * (c.TC * GW / 1024.0)) + 0.0109 * p.S);
+}
+
+static double est_resident(const PredictSizes& p) {
+  const int64_t G = 960 / p.RB;  // as the kernel's walkers
+  const double conf = lds_conflicts(p.T + 1);
+  const double walk = ceil_div((p.T + G - 1) / G, 2) * (0.378 + 0.068 * p.D + 0.0218 * conf);
+  const double sums = ceil_div(p.RB * p.K, 64) * (0.28 + p.R * (0.0145 + 0.00068 * conf));
+  return 6.1 + 0.586 * (p.T * p.H / 1024.0) + 0.069 * sums +
+         blocks_per_cu(p.n, p.RB) * (std::max(walk, sums) + 0.39 * (p.RB * p.S / 16384.0));
+}
+
+static double est_rows(const PredictSizes& p) {
+  const int64_t G = std::max<int64_t>(1, 1024 / p.RB);
+  const double conf = 0.00435 * lds_conflicts(p.TC + 1);
+  const double chunk = 0.687 + ceil_div((p.TC + G - 1) / G, 2) * (0.213 + 0.088 * p.D + 2 * conf) +
+                       ceil_div(p.RB * p.K, 1024) * p.TC / p.K * conf +
+                       0.254 * (p.TC * p.H / 1024.0);
+  return 7.0 + 0.216 * (p.RB * p.S / 16384.0) +
+         ceil_div(p.T, p.TC) * chunk * (1.0 + 0.52 * (blocks_per_cu(p.n, p.RB) - 1.0));
+}
+
+// a thread per (row, class), a dependent load a level: from the L2 while the
+// tables fit it, and past ~2^17 threads bound by their number
+static double est_heap(const PredictSizes& p) {
+  const double mb = (double)p.T * p.H * 12 / (1 << 20);
+  const double step = 0.24 + 0.33 * std::min(std::max((mb - 4.5) / 3.0, 0.0), 1.0);
+  return 5.0 + p.R * (p.D + 1) *
+                   std::max(step, (0.8 + 0.24 * p.D) * 1e-6 * (double)p.n * (double)p.K);
+}
+
+PredictPlan predict_plan(int64_t n, int64_t S, bool aligned16, int32_t K, int32_t D,
+                         int32_t n_rounds) {
+  PredictPlan o;
+  const int32_t H = (int32_t)((int64_t(2) << D) - 1);
+  if (predict_resident_plan(n, S, K, H, n_rounds, &o.RB, &o.lds))
+    o.kind = kPredictResident;
+  else if (predict_rows_plan(S, K, H, n_rounds, &o.RB, &o.TC, &o.lds))
+    o.kind = kPredictRows;
+  PredictPlan c;
+  c.kind = kPredictCols;
+  if (!aligned16 || !predict_cols_plan(S, K, D, n_rounds, &c.DX, &c.waves, &c.TC, &c.vt, &c.lds))
+    return o;
+  if (n > 255 * kColsRows && c.lds <= 80 * 1024) return c;
+  const PredictSizes p{n, S, K, n_rounds, (int64_t)n_rounds * K, H, D, o.RB, o.TC};
+  const double other = o.kind == kPredictResident ? est_resident(p)
+                       : o.kind == kPredictRows   ? est_rows(p)
+                                                  : est_heap(p);
+  // over several blocks a CU the estimates lean to the row blocks by 10% and
+  // to the column blocks by 5% where the trees are resident
+  const double lean = n <= 255 * kColsRows ? 1.0 : o.kind == kPredictResident ? 0.95 : 1.1;
+  return est_cols(p, c) < lean * other ? c : o;
 }
 
 // in-place row softmax over K logits: exp(x - max) / sum, sequential in k
