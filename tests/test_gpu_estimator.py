@@ -5,13 +5,15 @@ Bar: identical tree dicts (features, bins, leaf values as floats, sample
 counts), identical predictions and importances (bit-exact), for regression
 (config C1: 10k x 50, 32 bins, depth 5, 20 trees), softmax multiclass, era-aware DES, colsample subsets,
 warm start and save/load."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import clib, gbm, ops
 from tests.conftest import c1_data, print_case
-from warpgbm_amd import WarpGBM
+from warpgbm_amd import WarpGBM, _lib
 
 pytestmark = pytest.mark.gpu
 F32 = np.float32
@@ -601,6 +603,57 @@ def test_one_launch_levels_equal_level_chain(gpu, N, F, B, depth, classes):
     assert a.forest == b.forest
     assert sum(str(t).count("'feature'") for t in a.forest) > 0
     assert np.array_equal(bits(a.per_era_feature_importance_), bits(b.per_era_feature_importance_))
+
+
+def tile_launches(fit):
+    """Histogram tile launches of a level-wise fit (the level chain's; rounds of
+    one launch per level have none)."""
+    lib = _lib.load()
+    lib.wgbm_timer_reset()
+    lib.wgbm_timer_enable(1)
+    try:
+        fit()
+        torch.cuda.synchronize()
+    finally:
+        lib.wgbm_timer_enable(0)
+    ms, n = ctypes.c_double(), ctypes.c_int64()
+    _lib.check(lib.wgbm_timer_read(b"engine_hist_tiles", ctypes.byref(ms), ctypes.byref(n)),
+               "timer_read")
+    lib.wgbm_timer_reset()
+    return n.value
+
+
+# rows, features, bins, classes: one launch per level or the level chain (by the
+# turns of 256 workgroups, a CU each, that a launch takes)
+SMALL_ROUNDS = [
+    (12_288, 512, 5, 0, True), (12_288, 51, 5, 10, True),
+    (12_289, 511, 5, 0, True), (12_289, 512, 5, 0, False),
+    (16_384, 512, 32, 0, True), (16_385, 512, 32, 0, False), (16_385, 512, 63, 0, True),
+    (16_384, 51, 32, 10, False), (20_480, 51, 63, 10, True),
+    (20_480, 84, 5, 3, True), (20_480, 85, 5, 3, False), (20_480, 85, 16, 3, True),
+    (16_384, 85, 5, 3, True), (4097, 513, 10, 0, False), (20_481, 9, 10, 0, False),
+]
+
+
+@pytest.mark.parametrize("N,F,B,classes,small", SMALL_ROUNDS)
+def test_one_launch_levels_where_they_pay(gpu, N, F, B, classes, small):
+    """Which of a small one-era fit's rounds take one launch per level, on both
+    sides of each limit, and that the trees are those of the level chain."""
+    print_case("estimator", "one launch per level or chain", N, F, B, classes, small)
+    rng = np.random.default_rng(N + F)
+    X = rng.integers(0, B, (N, F)).astype(np.int8)
+    y = (X[:, 0] / B + 0.3 * rng.standard_normal(N)).astype(F32)
+    kw = dict(num_bins=B, max_depth=3, n_estimators=2, learning_rate=0.5, min_child_weight=3)
+    if classes:
+        kw["objective"] = "multiclass"
+        y = np.digitize(y, np.quantile(y, np.linspace(0, 1, classes + 1)[1:-1]))
+    m = WarpGBM(**kw)
+    assert (tile_launches(lambda: m.fit(X, y)) == 0) == small
+    chain = WarpGBM(**kw)
+    chain._engine_tuning = {8: 0}
+    assert tile_launches(lambda: chain.fit(X, y)) > 0
+    assert m.forest == chain.forest
+    assert "'feature'" in str(m.forest[0])
 
 
 @pytest.mark.parametrize("N,F,classes", [(20_481, 3, 0), (102_400, 3, 0), (102_401, 3, 0),

@@ -426,12 +426,13 @@ __global__ void complete_tables_kernel(const int32_t* feat, const int32_t* bin, 
 // one-era rounds of few rows, one launch per level (engine_small.hip): word
 // arrays [T * H] by heap index; ids: heap index of every row
 constexpr int64_t kSmallMaxRows = 20480;
-// (feature, tree) workgroups a launch may have: two on each CU at once; with
-// more, every level takes that many rounds of them.  Us per round, level chain
-// / one launch per level: 10000 rows x 50, depth 5 177 / 67; 20000 x 50 191 / 96;
-// 16000 x 200 227 / 106; 16000 x 500 241 / 179; 10000 x 50, 10 classes, depth 6 236 / 162; 16000 x
-// 100, 3 classes, 127 bins 497 / 279; past it 10000 x 100, 10 classes 261 / 287;
-// 16000 x 1000 248 / 314.
+// (feature, tree) workgroups a launch may have.  A CU holds one (two up to 2048
+// rows, whose rows take fewer registers), so every level takes a turn of them for
+// each 256, the trees' bookkeeping workgroups among them; see small_round_pays.
+// Us per round, level chain / one launch per level: 10000 rows x 50, depth 5 177 /
+// 67; 20000 x 50 191 / 96; 16000 x 200 227 / 106; 16000 x 500 241 / 179; 10000 x
+// 50, 10 classes, depth 6 236 / 162; 16000 x 100, 3 classes, 127 bins 497 / 279;
+// past it 10000 x 100, 10 classes 261 / 287; 16000 x 1000 248 / 314.
 constexpr int64_t kSmallMaxWork = 512;
 struct SmallArgs {
   int64_t n;
@@ -459,6 +460,7 @@ struct SmallArgs {
   TreeRecord rec;
 };
 bool small_round_fits(int64_t n, int32_t F, int32_t B, int32_t max_depth);
+bool small_round_pays(int64_t n, int32_t B, int32_t T, int32_t n_sel);
 int launch_small_level(SmallArgs a, int T, hipStream_t st);
 // column-block predictor: top levels evaluated whole, their words per tree
 // (padded), (row, class) sums per thread, rows per workgroup

@@ -683,7 +683,7 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
   WGBM_REQUIRE(rec.H == e->H, "engine_round: record has H=%d, expected %d", rec.H, e->H);
   const int T = c.n_trees, E = c.num_eras, F = c.n_feats, B = c.num_bins, D = c.max_depth;
   const int64_t N = c.n_rows;
-  if (e->small_fits && e->small_on && (int64_t)T * n_sel <= kSmallMaxWork)
+  if (e->small_fits && e->small_on && small_round_pays(N, B, T, n_sel))
     return small_round(e, target, pred, feat_sel, n_sel, rec, st);
   if (!e->part && !e->des_direct) {
     const int r = presize_levels(e);

@@ -359,7 +359,8 @@ __global__ __launch_bounds__(kSmThreads) void small_level_kernel(SmallArgs a) {
 static size_t small_lds(SmallArgs& a) {
   const int64_t nodes = int64_t(1) << a.depth, Bp = a.B | 1;
   // at most 16 copies (more take longer to add up than they save in
-  // conflicts) within 48 KB, so that two workgroups share a CU
+  // conflicts) within 48 KB (of what clearing and adding them up costs; a level
+  // whose cells alone take more has one copy)
   auto copies = [](int64_t words, int64_t bytes) {
     int lg = 4;
     while (lg > 0 && (words << lg) * bytes > 48 * 1024) --lg;
@@ -382,6 +383,23 @@ bool small_round_fits(int64_t n, int32_t F, int32_t B, int32_t max_depth) {
   const size_t h = small_lds(a);
   // (the last level's launch holds totals of 2^max_depth nodes, and no histogram)
   return h <= 128 * 1024 && ((int64_t(1) << max_depth) + 1) * 40 <= 128 * 1024;
+}
+
+// Whether one launch per level is faster than the level chain.  The chain's
+// launches take longer with more bins, and with more trees hardly longer; a
+// turn of these workgroups takes longer with more rows.  Level chain / one launch
+// per level, us per round of depth 5: up to 12288 rows it wins wherever it is
+// allowed (12288 x 51, 10 classes, 5 bins: 1.04 times); then at most two turns
+// (20480 x 400, 32 bins 1.3 times), but for few bins and a second turn of few
+// workgroups (20480 x 107, 3 classes, 5 bins 160 / 169; 128, 2 classes 158 / 165),
+// or three turns where bins or rows make up for them (20480 x 512, 63 bins 1.35
+// times, 32 bins 0.89; 16384 x 512, 32 bins 1.07, 10 classes 0.94).
+bool small_round_pays(int64_t n, int32_t B, int32_t T, int32_t n_sel) {
+  if ((int64_t)T * n_sel > kSmallMaxWork) return false;
+  const int64_t wgs = (int64_t)T * (n_sel + 1);
+  if (n <= 12288 || wgs <= 256) return true;
+  if (wgs <= 512) return !(n > 16384 && T > 1 && B <= 10 && wgs <= 384);
+  return B > 48 || (n <= 16384 && T <= 3 && B >= 32);
 }
 
 template <int RPT>
