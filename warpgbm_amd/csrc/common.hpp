@@ -192,6 +192,15 @@ __device__ __forceinline__ void wgbm_lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Order of the LDS accesses of one wave, whose lanes exchange data through words
+// that no other wave touches: the LDS serves a wave's accesses in order, so only
+// the compiler has to keep it (a barrier would also wait for the global stores).
+__device__ __forceinline__ void wgbm_wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Order between a wave's own agent-scope atomics: what it stored with them
 // before this has reached the agent's point of coherence before any memory
 // operation after it.  Enough to hand over data that is both written and read
@@ -261,6 +270,16 @@ __device__ __forceinline__ int64_t wgbm_wave_incl_scan_i64(int64_t x) {
   WGBM_SCANSTEP(0x142, 0xa)
   WGBM_SCANSTEP(0x143, 0xc)
 #undef WGBM_SCANSTEP
+  return x;
+}
+
+__device__ __forceinline__ uint32_t wgbm_wave_incl_scan_u32(uint32_t x) {
+  x += wgbm_dpp_u32<0x111, 0xf>(x);
+  x += wgbm_dpp_u32<0x112, 0xf>(x);
+  x += wgbm_dpp_u32<0x114, 0xf>(x);
+  x += wgbm_dpp_u32<0x118, 0xf>(x);
+  x += wgbm_dpp_u32<0x142, 0xa>(x);
+  x += wgbm_dpp_u32<0x143, 0xc>(x);
   return x;
 }
 

@@ -53,10 +53,13 @@ constexpr int kTransRows = 1024;
 // per column, threads per workgroup, most rows per row block (16-bit counts)
 constexpr int kQBuckets = 1024, kQSample = 1024, kQThreads = 1024, kQMaxRows = 65520;
 // columns from this length on take the two reads, shorter ones the transposed
-// copy, whose three launches cost less than the five here.  Times in us, copy
-// / two reads, at 32 bins: 30k x 50 smooth 125 / 155, with long tails and ties
-// 219 / 161; 100k x 100 155 / 186, 483 / 219; 200k x 100 199 / 229, 855 / 304;
-// 1M x 100 757 / 440, 4019 / 614.
+// copy, whose three launches cost less than the six here for smooth columns.
+// Times in us, copy / two reads, of smooth columns and of columns some of which
+// have long tails or ties, at 32 bins: 30k x 50 95 / 110, 189 / 117; 100k x 100
+// 124 / 121, 450 / 159; 131k x 1 113 / 117; 131k x 100 137 / 124, 568 / 183; 200k x
+// 100 168 / 135, 827 / 203; 1M x 100 728 / 325, 4011 / 638; at 5 bins 60k x 100 77
+// / 101, 258 / 113; 131k x 100 96 / 108, 469 / 134; 131k x 1 77 / 104; 200k x 100
+// 116 / 118, 687 / 159.
 constexpr int64_t kQuantileTwoReadRows = 1 << 17;
 int launch_quantile_two_reads(const float* X, int64_t n, int32_t F, int64_t xs, const float* q,
                               int32_t nq, float* edges, uint32_t* buf, int64_t ks,

@@ -10,7 +10,8 @@
 //               outliers nor a long tail stretch them;
 //   2. count    the first read: values per bucket, 16-bit counters in LDS,
 //               one lane per feature (a lane's counters all lie in its own
-//               bank: no conflicts), one partial table per row block;
+//               bank: no conflicts), one partial table per row block, then
+//               their sum;
 //   3. targets  the bucket of every target rank, numbered (slots), and a
 //               reference value for every slot in which several sample values
 //               are equal;
@@ -222,76 +223,102 @@ __global__ __launch_bounds__(kQThreads) void quantile_count_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// 3. targets: workgroup = 16 features of a chunk (a wave each after the sums)
+// the row blocks' counts added up: workgroup = 64 words of a chunk, a quarter of
+// the row blocks a wave
 // ---------------------------------------------------------------------------
+// Its own launch, over all CUs: added up by the few workgroups of the targets, 64
+// .. 196 tables one after the other took 61 .. 86 us of a call of 150 .. 230 (131k x
+// 1, 200k x 100), here 3 .. 6 us and 14 .. 16 for the targets.  Counts
+// [chunk][kQBuckets][64].
+__global__ __launch_bounds__(256) void quantile_sum_kernel(const uint32_t* __restrict__ part,
+                                                           int32_t nrb, int32_t nc,
+                                                           uint32_t* __restrict__ cnt) {
+  constexpr int W = kQBuckets / 2 * 64;
+  __shared__ uint32_t los[4][64], his[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int chunk = blockIdx.x / (W / 64), wd = blockIdx.x - chunk * (W / 64);
+  const uint32_t* p = part + (int64_t)chunk * W + wd * 64 + lane;
+  uint32_t lo = 0u, hi = 0u;
+  constexpr int RU = 16;  // row blocks in flight
+  for (int r0 = wave; r0 < nrb; r0 += 4 * RU) {
+    uint32_t x[RU];
+#pragma unroll
+    for (int k = 0; k < RU; ++k) {
+      const int r = r0 + 4 * k;
+      x[k] = p[(int64_t)(r < nrb ? r : nrb - 1) * nc * W];
+    }
+#pragma unroll
+    for (int k = 0; k < RU; ++k) {
+      const uint32_t v = r0 + 4 * k < nrb ? x[k] : 0u;
+      lo += v & 0xffffu;
+      hi += v >> 16;
+    }
+  }
+  los[wave][lane] = lo;
+  his[wave][lane] = hi;
+  __syncthreads();
+  if (wave < 2) {
+    const uint32_t(*s)[64] = wave ? his : los;
+    cnt[((int64_t)chunk * kQBuckets + 2 * wd + wave) * 64 + lane] =
+        s[0][lane] + s[1][lane] + s[2][lane] + s[3][lane];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 3. targets: workgroup = 16 features of a chunk
+// ---------------------------------------------------------------------------
+// A wave each after the loads: its words are its own, so nothing past them is a
+// barrier (each waited for the stores before it, a memory round trip: 23 us of
+// few features with 25 of them).
 __global__ __launch_bounds__(kQThreads) void quantile_targets_kernel(
-    const uint32_t* __restrict__ part, int64_t n, int32_t F, int32_t nrb,
-    const float* __restrict__ q, int32_t nq, const float2* __restrict__ map,
-    const float* __restrict__ sample, uint32_t* __restrict__ slot_map,
-    uint32_t* __restrict__ row_map, uint32_t* __restrict__ refs, uint32_t* __restrict__ slot_size,
-    uint32_t* __restrict__ slot_ref, uint8_t* __restrict__ tslot, int32_t* __restrict__ trank, int32_t* __restrict__ nslots) {
+    const uint32_t* __restrict__ counts, int64_t n, int32_t F, const float* __restrict__ q,
+    int32_t nq, const float2* __restrict__ map, const float* __restrict__ sample,
+    uint32_t* __restrict__ slot_map, uint32_t* __restrict__ row_map, uint32_t* __restrict__ refs,
+    uint32_t* __restrict__ slot_size, uint32_t* __restrict__ slot_ref,
+    uint8_t* __restrict__ tslot, int32_t* __restrict__ trank, int32_t* __restrict__ nslots) {
   constexpr int CS = kQBuckets + 1;  // odd row stride: the features' rows start in other banks
   __shared__ uint32_t cnt[16][CS];
   __shared__ uint8_t mark[16][kQBuckets];
-  const int nc = (F + 63) / 64;
   const int chunk = blockIdx.x >> 2, l0 = (blockIdx.x & 3) * 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int W = kQBuckets / 2 * 64;
+  const int fl = wave;
+  const int f = chunk * 64 + l0 + fl;
+  const bool on = f < F;
+  constexpr int SPER = kQSample / 64;
+  uint32_t sv[SPER];
+  const float2 m = map[on ? f : F - 1];
+#pragma unroll
+  for (int k = 0; k < SPER; ++k)
+    sv[k] = __float_as_uint(sample[(int64_t)(on ? f : F - 1) * kQSample + k * 64 + lane]);
   {
-    // counts of 16 features: thread (lane l0 + tid % 16, word group tid / 16)
-    const int l = tid & 15, wg = tid >> 4;
-    constexpr int NW = kQBuckets / 2 / (kQThreads / 16);
-    uint32_t lo[NW], hi[NW];
+    // counts of 16 features: thread (lane l0 + tid % 16, buckets tid / 16 ..)
+    const int l = tid & 15, b0 = tid >> 4;
+    constexpr int STEP = kQThreads / 16, NB = kQBuckets / STEP;
+    uint32_t x[NB];
 #pragma unroll
-    for (int k = 0; k < NW; ++k) lo[k] = hi[k] = 0u;
-    constexpr int RU = 4;  // row blocks in flight
-    for (int rb = 0; rb < nrb; rb += RU) {
-      uint32_t x[RU][NW];
+    for (int k = 0; k < NB; ++k)
+      x[k] = counts[((int64_t)chunk * kQBuckets + b0 + k * STEP) * 64 + l0 + l];
 #pragma unroll
-      for (int r = 0; r < RU; ++r) {
-        const int rr = rb + r < nrb ? rb + r : nrb - 1;
-        const uint32_t* p = part + ((int64_t)rr * nc + chunk) * W + l0 + l;
-#pragma unroll
-        for (int k = 0; k < NW; ++k) x[r][k] = p[(wg + k * (kQThreads / 16)) * 64];
-      }
-#pragma unroll
-      for (int r = 0; r < RU; ++r) {
-        if (rb + r >= nrb) break;  // uniform
-#pragma unroll
-        for (int k = 0; k < NW; ++k) {
-          lo[k] += x[r][k] & 0xffffu;
-          hi[k] += x[r][k] >> 16;
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      const int wd = wg + k * (kQThreads / 16);
-      cnt[l][2 * wd] = lo[k];
-      cnt[l][2 * wd + 1] = hi[k];
-    }
+    for (int k = 0; k < NB; ++k) cnt[l][b0 + k * STEP] = x[k];
     for (int i = tid; i < 16 * kQBuckets / 4; i += kQThreads)
       reinterpret_cast<uint32_t*>(&mark[0][0])[i] = 0u;
   }
   __syncthreads();
-  // from here on a wave owns feature f; its lane holds buckets PER * lane ..
+  // from here on a wave owns feature f; its lane holds buckets 64 k + lane
   constexpr int PER = kQBuckets / 64;
-  const int fl = wave;
-  const int f = chunk * 64 + l0 + fl;
-  const bool on = f < F;
-  uint32_t c[PER], sum = 0;
+  uint32_t c[PER];
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    c[k] = cnt[fl][lane * PER + k];
-    sum += c[k];
-  }
-  uint32_t base = (uint32_t)(wgbm_wave_incl_scan_i64((int64_t)sum) - sum);
+  for (int k = 0; k < PER; ++k) c[k] = cnt[fl][64 * k + lane];
+  {
+    uint32_t base = 0u;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    cnt[fl][lane * PER + k] = base;  // exclusive prefix
-    base += c[k];
+    for (int k = 0; k < PER; ++k) {
+      const uint32_t incl = wgbm_wave_incl_scan_u32(c[k]);
+      cnt[fl][64 * k + lane] = base + incl - c[k];  // exclusive prefix
+      base += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    }
   }
-  __syncthreads();
+  wgbm_wave_lds_order();
   const int nt = 2 * nq;
   const int64_t last = n - 1;
   constexpr int TPL = kSelMaxTargets / 64;  // targets per lane
@@ -313,23 +340,19 @@ __global__ __launch_bounds__(kQThreads) void quantile_targets_kernel(
     tb[j] = a;
     if (on) trank[(int64_t)f * kSelMaxTargets + t] = (int32_t)(r - (int64_t)cnt[fl][a]);
   }
-  __syncthreads();
-  uint32_t marks = 0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) marks |= (uint32_t)mark[fl][lane * PER + k] << k;
-  const int mine = __builtin_popcount(marks);
-  int s = (int)wgbm_wave_incl_scan_i64((int64_t)mine) - mine;
-  __syncthreads();
+  wgbm_wave_lds_order();
+  // slots: the marked buckets in order
+  int slots = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const bool m = (marks >> k) & 1u;
-    mark[fl][lane * PER + k] = m ? (uint8_t)s : (uint8_t)kQNone;
-    if (m) {
-      if (on) slot_size[(int64_t)f * 256 + s] = c[k];
-      ++s;
-    }
+    const bool mk = mark[fl][64 * k + lane] != 0;
+    const uint64_t bal = __ballot(mk);
+    const int s = slots + __builtin_popcountll(bal & ((1ull << lane) - 1ull));
+    mark[fl][64 * k + lane] = mk ? (uint8_t)s : (uint8_t)kQNone;
+    if (mk && on) slot_size[(int64_t)f * 256 + s] = c[k];
+    slots += __builtin_popcountll(bal);
   }
-  if (lane == 63 && on) nslots[f] = s;
+  if (lane == 0 && on) nslots[f] = slots;
   // four candidates a slot, each the last of a quarter of its sample values;
   // the one that most of the slot's sample values equal is its reference,
   // if any other does (a slot of distinct values needs none)
@@ -337,15 +360,9 @@ __global__ __launch_bounds__(kQThreads) void quantile_targets_kernel(
   uint32_t best[4] = {1u, 1u, 1u, 1u}, bref[4];  // of slots lane, lane + 64, ...
 #pragma unroll
   for (int j = 0; j < 4; ++j) bref[j] = 0xffffffffu;
-  constexpr int SPER = kQSample / 64;
-  uint32_t sv[SPER];
   int ss[SPER];
-  const float2 m = map[on ? f : F - 1];
-#pragma unroll
-  for (int k = 0; k < SPER; ++k)
-    sv[k] = __float_as_uint(sample[(int64_t)(on ? f : F - 1) * kQSample + k * 64 + lane]);
   for (int i = lane; i < 256; i += 64) votes[fl][i] = 0u;
-  __syncthreads();
+  wgbm_wave_lds_order();
 #pragma unroll
   for (int j = 0; j < TPL; ++j)
     if (tb[j] >= 0 && on)
@@ -364,11 +381,11 @@ __global__ __launch_bounds__(kQThreads) void quantile_targets_kernel(
 #pragma unroll
     for (int k = 0; k < SPER; ++k)
       if (ss[k] != kQNone && k % 4 == round) cand[fl][ss[k]] = sv[k];
-    __syncthreads();
+    wgbm_wave_lds_order();
 #pragma unroll
     for (int k = 0; k < SPER; ++k)
       if (ss[k] != kQNone && cand[fl][ss[k]] == sv[k]) atomicAdd(&votes[fl][ss[k]], 1u);
-    __syncthreads();
+    wgbm_wave_lds_order();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int i = j * 64 + lane;
@@ -379,12 +396,12 @@ __global__ __launch_bounds__(kQThreads) void quantile_targets_kernel(
         bref[j] = cand[fl][i];
       }
     }
-    __syncthreads();
+    wgbm_wave_lds_order();
   }
   // rows of the references: slot order within each quarter of the slots
   int row0 = 0;
   for (int i = lane; i < 256; i += 64) ref[fl][i] = 0xffffffffu;
-  __syncthreads();
+  wgbm_wave_lds_order();
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const uint64_t has = __ballot(bref[j] != 0xffffffffu);
@@ -395,7 +412,7 @@ __global__ __launch_bounds__(kQThreads) void quantile_targets_kernel(
     if (on) slot_ref[(int64_t)f * 256 + j * 64 + lane] = kept ? bref[j] : 0xffffffffu;
     row0 += __builtin_popcountll(has);
   }
-  __syncthreads();
+  wgbm_wave_lds_order();
   // the gather's tables: the reference row of every bucket, and the rows
   for (int wd = lane; wd < 256; wd += 64) {
     uint32_t x = 0;
@@ -737,12 +754,13 @@ int launch_quantile_two_reads(const float* X, int64_t n, int32_t F, int64_t xs, 
     return o;
   };
   const size_t o_sample = take((size_t)F * kQSample * 4), o_map = take((size_t)F * 8),
-               o_nan = take((size_t)F * 4), o_negz = take((size_t)F * 4), o_smap = take((size_t)nc * 256 * 64 * 4),
+               o_nan = take((size_t)F * 4), o_negz = take((size_t)F * 4),
+               o_smap = take((size_t)nc * 256 * 64 * 4),
                o_rmap = take((size_t)nc * 256 * 64 * 4), o_refs = take((size_t)nc * 128 * 64 * 4),
                o_size = take((size_t)F * 256 * 4), o_sref = take((size_t)F * 256 * 4),
                o_tslot = take((size_t)F * kSelMaxTargets),
                o_trank = take((size_t)F * kSelMaxTargets * 4), o_ns = take((size_t)F * 4),
-               o_gc = take((size_t)F * nrb * 4);
+               o_gc = take((size_t)F * nrb * 4), o_cnt = take((size_t)nc * kQBuckets * 64 * 4);
   uint32_t* part = (uint32_t*)scratch_get(st, part_b, 19);
   char* sm = (char*)scratch_get(st, off, 20);
   WGBM_REQUIRE(part && sm, "scratch allocation failed");
@@ -769,9 +787,12 @@ int launch_quantile_two_reads(const float* X, int64_t n, int32_t F, int64_t xs, 
   hipLaunchKernelGGL(quantile_count_kernel, grid, dim3(kQThreads), lds_count, st, X, n, F, xs,
                      (int32_t)rows_per, (int32_t)nrb, map, part, nanf, negz);
   WGBM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(quantile_targets_kernel, dim3((unsigned)(nc * 4)), dim3(kQThreads), 0, st,
-                     part, n, F, (int32_t)nrb, q, nq, map, sample, smap, rmap, refs, ssize, sref,
-                     tslot, trank, ns);
+  uint32_t* cnt = (uint32_t*)(sm + o_cnt);
+  hipLaunchKernelGGL(quantile_sum_kernel, dim3((unsigned)(nc * (kQBuckets / 2))), dim3(256), 0, st,
+                     part, (int32_t)nrb, (int32_t)nc, cnt);
+  WGBM_LAUNCH_CHECK();
+  hipLaunchKernelGGL(quantile_targets_kernel, dim3((unsigned)(nc * 4)), dim3(kQThreads), 0, st, cnt,
+                     n, F, q, nq, map, sample, smap, rmap, refs, ssize, sref, tslot, trank, ns);
   WGBM_LAUNCH_CHECK();
   hipLaunchKernelGGL(quantile_gather_kernel, grid, dim3(kQThreads), lds_gather, st, X, n, F, xs,
                      (int32_t)rows_per, (int32_t)nrb, map, rmap, refs, buf, ks, gc);
