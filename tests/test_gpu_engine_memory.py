@@ -1,0 +1,75 @@
+"""The level-wise engine's device memory: what its rounds need is taken when it
+is created (or tuned), so that a round allocates nothing."""
+import numpy as np
+import pytest
+import torch
+
+from tests.conftest import print_case
+from warpgbm_amd import device as D
+
+pytestmark = pytest.mark.gpu
+dev = torch.device("cuda:0")
+
+
+class Rounds:
+    """An engine on random codes in eras of equal length, and its first round."""
+
+    def __init__(self, N, F, B, E, depth, classes=0, level_bytes=0, tuning=()):
+        g = torch.Generator(device=dev)
+        g.manual_seed(N + F)
+        x8 = torch.randint(0, B, (N, F), generator=g, device=dev, dtype=torch.int8)
+        self.codes = D.codes_from_int8(x8, True, B)[0]
+        _, _, order, start = D.era_layout((np.arange(N) * E // N).astype(np.int32))
+        T, H = max(1, classes), (1 << (depth + 1)) - 1
+        signal = x8[:, 0].float() / B + 0.3 * torch.randn(N, generator=g, device=dev)
+        if classes:
+            cuts = torch.quantile(signal, torch.linspace(0, 1, classes + 1, device=dev)[1:-1])
+            self.target = torch.bucketize(signal, cuts).to(torch.int32)
+            self.start = torch.full((classes, N), -1.0, device=dev)
+        else:
+            self.target, self.start = signal, torch.zeros(N, device=dev)
+        self.sel = torch.arange(F, device=dev, dtype=torch.int32)
+        self.rec = dict(feat=torch.zeros((T, H), dtype=torch.int32, device=dev),
+                        bin=torch.zeros((T, H), dtype=torch.int32, device=dev),
+                        leaf=torch.zeros((T, H), device=dev),
+                        count=torch.zeros((T, H), dtype=torch.int64, device=dev),
+                        gain=torch.zeros((T, H, E), device=dev))
+        self.pred = self.start.clone()
+        self.eng = D.Engine(self.codes, torch.from_numpy(order).to(dev),
+                            torch.from_numpy(start).to(dev), B, E, depth, T,
+                            1 if classes else 0, 20.0, 0.0, 1e-6, 0.1, level_bytes)
+        for key, value in tuning:
+            self.eng.set_tuning(key, value)
+
+    def round(self):
+        self.pred.copy_(self.start)
+        self.eng.round(self.target, self.pred, self.sel, self.rec)
+        torch.cuda.synchronize()
+        return [self.pred.clone()] + [self.rec[k].clone() for k in sorted(self.rec)]
+
+
+def free_bytes():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info(dev)[0]
+
+
+# rows, features, bins, eras, depth, classes, level bytes, tuning
+ERA_ENGINES = [
+    # 12 nodes of three class trees in chunks of 8 and 4
+    (80_000, 600, 127, 2, 3, 3, 150_000_000, ()),
+    (80_000, 600, 127, 2, 4, 0, 0, ()),
+]
+
+
+@pytest.mark.parametrize("case", ERA_ENGINES, ids=[str(c) for c in ERA_ENGINES])
+def test_era_rounds_allocate_nothing(gpu, case):
+    """Direct era path with tiled levels, also in chunks that do not divide a
+    level: the first round of an engine takes no device memory."""
+    print_case("engine memory", "era rounds", *case)
+    first = Rounds(*case).round()  # (kernels are loaded by now)
+    r = Rounds(*case)
+    before = free_bytes()
+    out = r.round()
+    assert free_bytes() == before
+    assert all(torch.equal(a, b) for a, b in zip(out, first))
+    assert int((r.rec["feat"] >= 0).sum()) > 0

@@ -533,7 +533,8 @@ static int level_plan(Engine* e, int d, LevelPlan* lp) {
 }
 
 // direct era levels of few large segments (era_level_tiles): the tiles of nc
-// (tree, node)s, the level split into n_chunk such runs
+// (tree, node)s, the level split into n_chunk such runs (the last may be shorter:
+// its tiles have the rows of the others', so they never need more room)
 static void era_tile_sizes(const Engine* e, int64_t nc, int n_chunk, LevelPlan* lp) {
   const int64_t TN = (int64_t)e->c.n_trees * e->c.n_rows;
   lp->n_list = (int32_t)(nc * e->c.num_eras);
@@ -820,7 +821,7 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
         if (use_tiles) {
           // few large segments: split over tiles, then scanned from the tiles
           LevelPlan lp;
-          r = era_tile_plan(e, nc, (n_tn + nc - 1) / nc, &lp);
+          r = era_tile_plan(e, nc, (int)((n_tn + e->nc_max - 1) / e->nc_max), &lp);
           if (r) return r;
           if (!planned) {  // (else by the previous level's scan)
             hipLaunchKernelGGL(plan_tiles_kernel<true>, dim3(1), dim3(1024), 0, st,
