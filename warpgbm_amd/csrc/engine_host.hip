@@ -149,6 +149,7 @@ static int dalloc(Engine* e, T** p, int64_t n) {
   if (err != hipSuccess) {
     wgbm_set_error("engine: hipMalloc of %lld bytes failed: %s", (long long)(n * sizeof(T)),
                    hipGetErrorString(err));
+    (void)hipGetLastError();  // (reported here: not again by the next launch)
     return WGBM_ENOMEM;
   }
   e->allocs.push_back(q);
@@ -466,6 +467,7 @@ static int ensure_partials(Engine* e, int64_t max_tiles) {
         break;
       }
     e->part = nullptr;
+    e->part_words = 0;  // nothing holds tiles if the allocation below fails
   }
   int r = dalloc(e, &e->part, words);
   if (r) return r;
@@ -488,6 +490,7 @@ static int ensure_tiles(Engine* e, int64_t max_tiles) {
           break;
         }
       e->htiles = nullptr;
+      e->max_htiles = 0;
     }
     r = dalloc(e, &e->htiles, max_tiles);
     if (r) return r;
@@ -573,7 +576,6 @@ static int presize_levels(Engine* e) {
     if (r != WGBM_ENOMEM) return r;
     // no room for the tiles' partials: every level takes the per-segment
     // kernels, which need none
-    (void)hipGetLastError();
     e->era_tiles = false;
     return 0;
   }
