@@ -43,9 +43,13 @@ class Rounds:
             self.eng.set_tuning(key, value)
 
     def round(self):
+        """A round from the start, and the device memory that it took."""
         self.pred.copy_(self.start)
+        before = free_bytes()
         self.eng.round(self.target, self.pred, self.sel, self.rec)
-        torch.cuda.synchronize()
+        return before - free_bytes()
+
+    def out(self):
         return [self.pred.clone()] + [self.rec[k].clone() for k in sorted(self.rec)]
 
 
@@ -54,25 +58,55 @@ def free_bytes():
     return torch.cuda.mem_get_info(dev)[0]
 
 
+def fill_memory():
+    """All device memory but about 200 MB (what was freed before comes back late)."""
+    hog = []
+    while free_bytes() > 250_000_000:
+        hog.append(torch.empty(free_bytes() - 200_000_000, dtype=torch.uint8, device=dev))
+    return hog
+
+
 # rows, features, bins, eras, depth, classes, level bytes, tuning
 ERA_ENGINES = [
     # 12 nodes of three class trees in chunks of 8 and 4
     (80_000, 600, 127, 2, 3, 3, 150_000_000, ()),
     (80_000, 600, 127, 2, 4, 0, 0, ()),
+    # smaller tiles, and int8 codes at few bins (tiled from shorter segments on)
+    (180_000, 300, 127, 3, 3, 0, 0, ((1, 256),)),
+    (190_000, 2000, 7, 3, 5, 0, 0, ((2, 0), (1, 256))),
 ]
 
 
 @pytest.mark.parametrize("case", ERA_ENGINES, ids=[str(c) for c in ERA_ENGINES])
 def test_era_rounds_allocate_nothing(gpu, case):
     """Direct era path with tiled levels, also in chunks that do not divide a
-    level: the first round of an engine takes no device memory."""
+    level and with tile sizes set after the engine was created: the first round
+    of an engine takes no device memory."""
     print_case("engine memory", "era rounds", *case)
-    first = Rounds(*case).round()  # (kernels are loaded by now)
+    first = Rounds(*case)
+    first.round()  # (kernels are loaded by now)
     r = Rounds(*case)
-    before = free_bytes()
-    out = r.round()
-    assert free_bytes() >= before
-    assert all(torch.equal(a, b) for a, b in zip(out, first))
+    assert r.round() <= 0  # (memory freed earlier may come back meanwhile)
+    assert all(torch.equal(a, b) for a, b in zip(r.out(), first.out()))
+    assert int((r.rec["feat"] >= 0).sum()) > 0
+
+
+def test_era_tiles_without_room(gpu):
+    """A tile size whose buffers find no memory: the era levels go without tiles,
+    and grow the same trees."""
+    case = (400_000, 1000, 127, 7, 3)
+    print_case("engine memory", "era tiles without room", *case)
+    want = Rounds(*case)
+    want.round()
+    want = want.out()
+    r = Rounds(*case)
+    torch.cuda.empty_cache()
+    hog = fill_memory()
+    r.eng.set_tuning(1, 256)
+    r.round()
+    del hog
+    torch.cuda.empty_cache()
+    assert all(torch.equal(a, b) for a, b in zip(r.out(), want))
     assert int((r.rec["feat"] >= 0).sum()) > 0
 
 
@@ -83,16 +117,17 @@ def test_round_after_failed_growth(gpu):
     then, with the trees of an engine that never failed."""
     case = (1_000_000, 1000, 127, 1, 6, 0, 7_000_000)
     print_case("engine memory", "failed growth", *case)
-    want = Rounds(*case).round()
+    want = Rounds(*case)
+    want.round()
+    want = want.out()
     r = Rounds(*case)
     torch.cuda.empty_cache()
-    hog = []
-    while free_bytes() > 250_000_000:  # (what was freed before comes back late)
-        hog.append(torch.empty(free_bytes() - 200_000_000, dtype=torch.uint8, device=dev))
+    hog = fill_memory()
     for _ in range(2):
         with pytest.raises(_lib.WgbmError, match="hipMalloc"):
             r.round()
     del hog
     torch.cuda.empty_cache()
-    assert all(torch.equal(a, b) for a, b in zip(r.round(), want))
+    r.round()
+    assert all(torch.equal(a, b) for a, b in zip(r.out(), want))
     assert int((r.rec["feat"] >= 0).sum()) > 0

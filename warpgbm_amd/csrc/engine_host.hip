@@ -173,6 +173,7 @@ void engine_destroy(Engine* e) {
 }
 
 static int presize_levels(Engine* e);
+static int resize_era_tiles(Engine* e);
 
 int engine_create(Engine** out, const EngineConfig& cfg) {
   WGBM_REQUIRE(cfg.n_rows > 0 && cfg.n_rows < (int64_t(1) << 31), "engine: n_rows out of range");
@@ -407,7 +408,7 @@ int engine_set_tuning(Engine* e, int key, int64_t value) {
                  "hist tile rows must be 0 or in [256, %d]", WGBM_MAX_TILE_ROWS);
     e->hist_tile_rows = value;
     e->root_tiles_ready = false;  // the root plan depends on the tile rows
-    return 0;
+    return resize_era_tiles(e);
   }
   if (key == 5) {
     WGBM_REQUIRE(value == 0 || value == 1, "one-era root path must be 0 or 1");
@@ -427,7 +428,7 @@ int engine_set_tuning(Engine* e, int key, int64_t value) {
   if (key == 2) {
     WGBM_REQUIRE(value == 0 || value == 1, "era code layout must be 0 or 1");
     e->des_codes = (int)value;
-    return 0;
+    return resize_era_tiles(e);
   }
   if (key == 3) {
     WGBM_REQUIRE(value == 0 || value == 1, "one-era level scan must be 0 or 1");
@@ -587,6 +588,14 @@ static int presize_levels(Engine* e) {
     mt = std::max(mt, lp.max_tiles);
   }
   return mt > 0 ? ensure_tiles(e, mt) : 0;
+}
+
+// a knob of the direct era path's tiles was set: their buffers for the new sizes,
+// so that the rounds still allocate nothing (or no tiles where there is no room)
+static int resize_era_tiles(Engine* e) {
+  if (!e->des_direct) return 0;
+  e->era_tiles = true;
+  return presize_levels(e);
 }
 
 // histogram tiles of one chunk of a level (n_list keys, the chunk's present
