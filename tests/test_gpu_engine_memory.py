@@ -36,11 +36,15 @@ class Rounds:
                         count=torch.zeros((T, H), dtype=torch.int64, device=dev),
                         gain=torch.zeros((T, H, E), device=dev))
         self.pred = self.start.clone()
-        self.eng = D.Engine(self.codes, torch.from_numpy(order).to(dev),
-                            torch.from_numpy(start).to(dev), B, E, depth, T,
-                            1 if classes else 0, 20.0, 0.0, 1e-6, 0.1, level_bytes)
+        order, start = torch.from_numpy(order).to(dev), torch.from_numpy(start).to(dev)
+        self.args = (self.codes, order, start, B, E, depth, T, 1 if classes else 0, 20.0, 0.0,
+                     1e-6, 0.1)
+        self.create(level_bytes)
         for key, value in tuning:
             self.eng.set_tuning(key, value)
+
+    def create(self, level_bytes):
+        self.eng = D.Engine(*self.args, level_bytes)
 
     def round(self):
         """A round from the start, and the device memory that it took."""
@@ -89,6 +93,27 @@ def test_era_rounds_allocate_nothing(gpu, case):
     assert r.round() <= 0  # (memory freed earlier may come back meanwhile)
     assert all(torch.equal(a, b) for a, b in zip(r.out(), first.out()))
     assert int((r.rec["feat"] >= 0).sum()) > 0
+
+
+def test_era_tiles_within_the_level_budget(gpu):
+    """The tiles' partials of a level are at most the level budget: with 100 MB the
+    engine takes less than twice that besides its per-row arrays (a level of 40 (node,
+    era)s and 342 row tiles would take 397 MB more), and grows the same trees."""
+    case = (350_000, 1000, 127, 10, 6)
+    print_case("engine memory", "era tiles within the budget", *case)
+    big = Rounds(*case)
+    big.round()
+    budget = 100_000_000
+    r = Rounds(*case, 0, budget)
+    torch.cuda.empty_cache()
+    r.eng.close()
+    before = free_bytes()
+    r.create(budget)
+    taken = before - free_bytes()
+    assert taken < 2 * budget + 150 * 350_000 + (64 << 20)
+    r.round()
+    assert all(torch.equal(a, b) for a, b in zip(r.out(), big.out()))
+    assert int((r.rec["feat"] >= 0).sum()) > 20
 
 
 def test_era_tiles_without_room(gpu):

@@ -23,6 +23,24 @@ def bits(a):
     return np.asarray(a, dtype=F32).view(np.uint32)
 
 
+def tile_launches(fit):
+    """Histogram tile launches of a level-wise fit (the level chain's; rounds of
+    one launch per level have none)."""
+    lib = _lib.load()
+    lib.wgbm_timer_reset()
+    lib.wgbm_timer_enable(1)
+    try:
+        fit()
+        torch.cuda.synchronize()
+    finally:
+        lib.wgbm_timer_enable(0)
+    ms, n = ctypes.c_double(), ctypes.c_int64()
+    _lib.check(lib.wgbm_timer_read(b"engine_hist_tiles", ctypes.byref(ms), ctypes.byref(n)),
+               "timer_read")
+    lib.wgbm_timer_reset()
+    return n.value
+
+
 def oracle_codes(model, X):
     """Codes the oracle bins X to, with edges the oracle computes itself."""
     edges = ops.quantile_edges(X, model.num_bins)
@@ -256,16 +274,17 @@ def test_era_des_bins_and_blocks_bit_exact(gpu, E, B):
     assert np.array_equal(bits(m.predict(X)), bits(ref.predict_codes(X)))
 
 
-@pytest.mark.parametrize("B,N,F,classes,chunked", [
-    (2, 40_000, 40, 0, False), (7, 27_000, 70, 0, False), (16, 9_001, 130, 0, False),
-    (17, 9_001, 65, 3, False), (32, 12_345, 260, 0, True), (64, 9_001, 129, 0, False),
-    (65, 9_001, 66, 0, False), (127, 12_345, 64, 0, False)])
-def test_era_des_tiled_levels_bit_exact(gpu, B, N, F, classes, chunked):
+@pytest.mark.parametrize("B,N,F,classes,level_bytes", [
+    (2, 40_000, 40, 0, 0), (7, 27_000, 70, 0, 0), (16, 9_001, 130, 0, 0), (17, 9_001, 65, 3, 0),
+    (32, 12_345, 260, 0, 3_000_000), (32, 12_345, 260, 0, 1_600_000), (64, 9_001, 129, 0, 0),
+    (65, 9_001, 66, 0, 0), (127, 12_345, 64, 0, 0)])
+def test_era_des_tiled_levels_bit_exact(gpu, B, N, F, classes, level_bytes):
     """Few large eras: the shallow levels histogram (node, era) segments over
     row tiles and scan them from the tiles, the deeper ones take the per-segment
     kernels; every instance of the scan, uneven eras (a dead and an empty-node
-    one among them), class trees, codes outside the bins, level chunks."""
-    print_case("estimator", "DES tiled levels", B, N, F, classes, chunked)
+    one among them), class trees, codes outside the bins, level chunks of a few
+    nodes, and a level budget that the tiles' partials would exceed (no tiles)."""
+    print_case("estimator", "DES tiled levels", B, N, F, classes, level_bytes)
     rng = np.random.default_rng(B)
     sizes = np.array([N - N // 3 - 15, N // 3, 15])
     era = np.repeat(np.arange(3), sizes)
@@ -280,9 +299,9 @@ def test_era_des_tiled_levels_bit_exact(gpu, B, N, F, classes, chunked):
     else:
         y = score.astype(F32)
     m = WarpGBM(colsample_bytree=0.8, random_state=3, **kw)
-    if chunked:
-        m._engine_level_bytes = 600_000  # a few nodes per chunk
-    m.fit(X, y, era_id=era)
+    m._engine_level_bytes = level_bytes
+    tiled = tile_launches(lambda: m.fit(X, y, era_id=era)) > 0
+    assert tiled == (level_bytes != 1_600_000)
     ref = gbm.Forest(**kw).fit_codes(X, y, era_id=era, feat_sets=m.feature_subsets_,
                                      hist=clib.hist_exact_q, scan=clib.split_scan_q)
     for i, (a, b) in enumerate(zip(m.forest, ref.forest)):
@@ -603,24 +622,6 @@ def test_one_launch_levels_equal_level_chain(gpu, N, F, B, depth, classes):
     assert a.forest == b.forest
     assert sum(str(t).count("'feature'") for t in a.forest) > 0
     assert np.array_equal(bits(a.per_era_feature_importance_), bits(b.per_era_feature_importance_))
-
-
-def tile_launches(fit):
-    """Histogram tile launches of a level-wise fit (the level chain's; rounds of
-    one launch per level have none)."""
-    lib = _lib.load()
-    lib.wgbm_timer_reset()
-    lib.wgbm_timer_enable(1)
-    try:
-        fit()
-        torch.cuda.synchronize()
-    finally:
-        lib.wgbm_timer_enable(0)
-    ms, n = ctypes.c_double(), ctypes.c_int64()
-    _lib.check(lib.wgbm_timer_read(b"engine_hist_tiles", ctypes.byref(ms), ctypes.byref(n)),
-               "timer_read")
-    lib.wgbm_timer_reset()
-    return n.value
 
 
 # rows, features, bins, classes: one launch per level or the level chain (by the

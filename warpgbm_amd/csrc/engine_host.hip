@@ -60,6 +60,7 @@ struct Engine {
   unsigned long long* part = nullptr;
   uint32_t* abs_part = nullptr;
   int64_t part_words = 0;
+  int64_t budget = 0;  // bytes of the per-level buffers (level_bytes)
   int64_t* hq[2] = {nullptr, nullptr};
   int32_t* hc[2] = {nullptr, nullptr};
   float* crit = nullptr;         // E > 1: per-candidate era-mean gain [tn][n_sel*(B-1)]
@@ -134,6 +135,11 @@ struct Engine {
   size_t arena_size = 0, arena_used = 0;
 };
 
+// bytes of one histogram tile's partial
+static int64_t tile_part_bytes(const Engine* e) {
+  return (int64_t)e->n_chunks * kHistSlots * e->V * e->c.num_bins * 8;
+}
+
 template <typename T>
 static int dalloc(Engine* e, T** p, int64_t n) {
   if (n < 1) n = 1;
@@ -174,6 +180,7 @@ void engine_destroy(Engine* e) {
 
 static int presize_levels(Engine* e);
 static int resize_era_tiles(Engine* e);
+static int64_t era_tiles_max(const Engine* e);
 
 int engine_create(Engine** out, const EngineConfig& cfg) {
   WGBM_REQUIRE(cfg.n_rows > 0 && cfg.n_rows < (int64_t(1) << 31), "engine: n_rows out of range");
@@ -232,6 +239,7 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
                           W * (4 + F * (B - 1) * 9) + F * (B - 1) * 8
                     : 2 * E * F * B * 12 + (E > 1 ? F * (B - 1) * 8 : 0);
   const int64_t budget = cfg.level_bytes > 0 ? cfg.level_bytes : (int64_t)4 << 30;
+  e->budget = budget;
   if (T * hist_nodes_max * per_node <= budget) {
     e->nc_max = T * hist_nodes_max;
   } else {
@@ -247,13 +255,22 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
     // partition words; nodes: flags, shifts, maxima, picks, leaf values and
     // the chosen split's per-era gains; the pair codes; 64 MiB of slack
     const int64_t keys = e->n_keys_max, tn = T * nodes_max;
-    const int64_t pcodes = (e->des_direct && B <= 7) ? N * pair_stride((int32_t)F) : 0;
+    if (e->des_direct && B <= 7 && N * pair_stride((int32_t)F) <= (int64_t)0xffffffffll)
+      e->pstride = pair_stride((int32_t)F);
+    const int64_t pcodes = N * e->pstride;
     const int64_t small =
         E == 1 && small_round_fits(N, (int32_t)F, (int32_t)B, D) ? T * N * 4 + T * e->H * 40 : 0;
-    const int64_t need = small + e->nc_max * per_node + T * N * 29 + keys * 132 + tn * 76 + tn * E * 4 +
-                         pcodes + ((int64_t)64 << 20);
+    int64_t need = small + e->nc_max * per_node + T * N * 29 + keys * 132 + tn * 76 + tn * E * 4 +
+                   pcodes + ((int64_t)64 << 20);
     size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && (size_t)need > free_b) {
+    const bool known = hipMemGetInfo(&free_b, &total_b) == hipSuccess;
+    if (e->des_direct) {
+      // the era levels' tiles, which can be done without
+      const int64_t tiles = era_tiles_max(e) * (tile_part_bytes(e) + (int64_t)sizeof(Tile));
+      if (known && (size_t)(need + tiles) > free_b) e->era_tiles = false;
+      else need += tiles;
+    }
+    if (known && (size_t)need > free_b) {
       wgbm_set_error("engine: needs about %.1f GiB of device memory (max_depth=%d, %d eras, "
                      "%lld rows x %d trees), %.1f GiB free; reduce max_depth or the data",
                      need / 1073741824.0, D, (int)E, (long long)N, (int)T,
@@ -290,10 +307,7 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
     E_ALLOC(e->sgain, des_stage_words(e->nc_max, (int32_t)W, F * (B - 1)));
     E_ALLOC(e->sdir, des_stage_words(e->nc_max, (int32_t)W, F * (B - 1)));
     E_ALLOC(e->local_of, F);
-    if (B <= 7 && N * pair_stride((int32_t)F) <= (int64_t)0xffffffffll) {
-      e->pstride = pair_stride((int32_t)F);
-      E_ALLOC(e->pcodes, N * e->pstride);
-    }
+    if (e->pstride) E_ALLOC(e->pcodes, N * e->pstride);
     E_ALLOC(e->alive, e->nc_max * W);
     E_ALLOC(e->wg_agree, e->nc_max * ((F * (B - 1) + 255) / 256));
     E_ALLOC(e->wg_key, e->nc_max * ((F * (B - 1) + 255) / 256));
@@ -456,7 +470,7 @@ static int64_t pick_tile_rows(const Engine* e, int64_t rows_bound, int64_t least
 }
 
 static int ensure_partials(Engine* e, int64_t max_tiles) {
-  const int64_t words = max_tiles * e->n_chunks * kHistSlots * e->V * e->c.num_bins;
+  const int64_t words = max_tiles * (tile_part_bytes(e) / 8);
   if (words <= e->part_words) return 0;
   if (e->part) {
     // partial buffers are only reused within the stream; grow after a sync
@@ -553,11 +567,27 @@ static int era_tile_plan(Engine* e, int64_t nc, int n_chunk, LevelPlan* lp) {
 }
 
 // whether depth d of the direct era path takes tiles: by the mean rows of a
-// (node, era) segment (see kEraTileRows)
-static bool era_level_tiles(const Engine* e, int d) {
+// (node, era) segment (see kEraTileRows), and while the tiles' partials stay
+// within the level budget, of which the other level buffers may take as much
+// again.  sizes (optional): those of the depth's first chunk.
+static bool era_level_tiles(const Engine* e, int d, LevelPlan* sizes = nullptr) {
   if (!e->era_tiles) return false;
-  const int64_t rows = e->pcodes && e->des_codes == 1 ? kEraTileRowsPair : kEraTileRows;
-  return e->c.n_rows >= rows * (int64_t(1) << d) * e->c.num_eras;
+  const int64_t rows = e->pstride && e->des_codes == 1 ? kEraTileRowsPair : kEraTileRows;
+  if (e->c.n_rows < rows * (int64_t(1) << d) * e->c.num_eras) return false;
+  const int64_t n_tn = (int64_t)e->c.n_trees << d, nc = std::min(e->nc_max, n_tn);
+  LevelPlan lp;
+  era_tile_sizes(e, nc, (int)((n_tn + nc - 1) / nc), &lp);
+  if (sizes) *sizes = lp;
+  return lp.max_tiles * tile_part_bytes(e) <= e->budget;
+}
+
+// most tiles of a depth of the direct era path
+static int64_t era_tiles_max(const Engine* e) {
+  int64_t mt = 0;
+  LevelPlan lp;
+  for (int d = 0; d < e->c.max_depth; ++d)
+    if (era_level_tiles(e, d, &lp)) mt = std::max(mt, lp.max_tiles);
+  return mt;
 }
 
 // the tile buffers of every level a round histograms, sized once, with the
@@ -567,12 +597,7 @@ static bool era_level_tiles(const Engine* e, int d) {
 static int presize_levels(Engine* e) {
   int64_t mt = 0;
   if (e->des_direct) {
-    for (int d = 0; d < e->c.max_depth && era_level_tiles(e, d); ++d) {
-      const int64_t n_tn = (int64_t)e->c.n_trees << d, nc = std::min(e->nc_max, n_tn);
-      LevelPlan lp;
-      era_tile_sizes(e, nc, (int)((n_tn + nc - 1) / nc), &lp);
-      mt = std::max(mt, lp.max_tiles);
-    }
+    mt = era_tiles_max(e);
     const int r = mt > 0 ? ensure_tiles(e, mt) : 0;
     if (r != WGBM_ENOMEM) return r;
     // no room for the tiles' partials: every level takes the per-segment
