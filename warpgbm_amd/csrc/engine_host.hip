@@ -108,6 +108,7 @@ struct Engine {
   int32_t* root_hn = nullptr;
   int64_t root_tiles_cap = 0;
   bool root_tiles_ready = false;
+  // (E > 32, direct path)
   uint32_t* alive = nullptr;    // [tn][W] segments that can hold a split, W = ceil(E/32)
   double* bsum = nullptr;       // [tn][W][n_sel*(B-1)] era-block gain sums
   int8_t* bdir = nullptr;       // [tn][W][n_sel*(B-1)] era-block direction sums (|.| <= 32)
@@ -236,7 +237,7 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
   const int64_t W = (E + kDesEraBlock - 1) / kDesEraBlock;
   const int64_t per_node =
       e->des_direct ? des_stage_words(1, (int32_t)W, F * (B - 1)) * 5 +
-                          W * (4 + F * (B - 1) * 9) + F * (B - 1) * 8
+                          (W > 1 ? W * (4 + F * (B - 1) * 9) : 0) + F * (B - 1) * 8
                     : 2 * E * F * B * 12 + (E > 1 ? F * (B - 1) * 8 : 0);
   const int64_t budget = cfg.level_bytes > 0 ? cfg.level_bytes : (int64_t)4 << 30;
   e->budget = budget;
@@ -308,11 +309,13 @@ int engine_create(Engine** out, const EngineConfig& cfg) {
     E_ALLOC(e->sdir, des_stage_words(e->nc_max, (int32_t)W, F * (B - 1)));
     E_ALLOC(e->local_of, F);
     if (e->pstride) E_ALLOC(e->pcodes, N * e->pstride);
-    E_ALLOC(e->alive, e->nc_max * W);
     E_ALLOC(e->wg_agree, e->nc_max * ((F * (B - 1) + 255) / 256));
     E_ALLOC(e->wg_key, e->nc_max * ((F * (B - 1) + 255) / 256));
-    E_ALLOC(e->bsum, e->nc_max * W * F * (B - 1));
-    E_ALLOC(e->bdir, e->nc_max * W * F * (B - 1));
+    if (W > 1) {  // (one block of eras is summed by the pick itself)
+      E_ALLOC(e->alive, e->nc_max * W);
+      E_ALLOC(e->bsum, e->nc_max * W * F * (B - 1));
+      E_ALLOC(e->bdir, e->nc_max * W * F * (B - 1));
+    }
   }
   E_ALLOC(e->dirbit, T * N);
   E_ALLOC(e->keyp[0], T * N);
@@ -1131,7 +1134,7 @@ int engine_round(Engine* e, const void* target, float* pred, const int32_t* feat
     nx.node_shift_next = e->node_shift[nxt];
     // the next era level's live-era masks, when it runs whole: written by
     // node_scan_kernel (no des_alive_kernel launch there)
-    const bool next_alive = d + 1 < D && e->des_direct && 2 * (int64_t)n_tn <= e->nc_max;
+    const bool next_alive = d + 1 < D && e->alive && 2 * (int64_t)n_tn <= e->nc_max;
     nx.alive_next = nullptr;
     nx.mcw = mcw;
     if (d < D && one_wg) {
