@@ -71,18 +71,22 @@ def test_c1_regression_bit_exact(gpu):
     assert np.corrcoef(p, y)[0, 1] > 0.9
 
 
+@pytest.mark.parametrize("small", [0, 1])
 @pytest.mark.parametrize("B", [5, 8, 10, 16, 64])
-def test_one_era_bin_counts_bit_exact(gpu, B):
+def test_one_era_bin_counts_bit_exact(gpu, B, small):
     """The one-era split step's compile-time bin counts (10 is the
-    estimator's default) grow the oracle's trees: regression on 6000 rows
-    and a 3-class softmax, depth 4."""
-    print_case("estimator", "one-era bin count", B)
+    estimator's default) grow the oracle's trees, in the level chain and, as the
+    small rounds' runtime bin count, with one launch per level: regression on 6000
+    rows and a 3-class softmax, depth 4."""
+    print_case("estimator", "one-era bin count, small", B, small)
     rng = np.random.default_rng(40 + B)
     N, F = 6000, 12
     X = rng.standard_normal((N, F)).astype(F32)
     y = (X[:, 0] - 0.5 * X[:, 3] ** 2 + 0.1 * rng.standard_normal(N)).astype(F32)
     kw = dict(num_bins=B, max_depth=4, n_estimators=3, learning_rate=0.3, min_child_weight=5)
-    m = WarpGBM(**kw).fit(X, y)
+    m = WarpGBM(**kw)
+    m._engine_tuning = {8: small}
+    assert (tile_launches(lambda: m.fit(X, y)) == 0) == bool(small)
     codes = oracle_codes(m, X)
     ref = gbm.Forest(**kw).fit_codes(codes, y)
     for i, (a, b) in enumerate(zip(m.forest, ref.forest)):
@@ -91,7 +95,9 @@ def test_one_era_bin_counts_bit_exact(gpu, B):
     labels = (X[:, 1] > 0).astype(np.int64) + (X[:, 2] > 0.5)
     kw = dict(objective="multiclass", num_bins=B, max_depth=4, n_estimators=2,
               learning_rate=0.3, min_child_weight=5)
-    m = WarpGBM(**kw).fit(X, labels)
+    m = WarpGBM(**kw)
+    m._engine_tuning = {8: small}
+    assert (tile_launches(lambda: m.fit(X, labels)) == 0) == bool(small)
     codes = oracle_codes(m, X)
     ref = gbm.Forest(**kw).fit_codes(codes, labels)
     for i, (a, b) in enumerate(zip(m.forest, ref.forest)):
@@ -575,17 +581,21 @@ def test_des_leaf_when_max_agreement_candidates_fail_min_split_gain(gpu):
         assert np.array_equal(bits(m.predict(X)), bits(ref.predict_codes(X)))
 
 
-@pytest.mark.parametrize("level_bytes", [0, 1])
-def test_chunked_levels_regression_bit_exact(gpu, level_bytes):
+@pytest.mark.parametrize("level_bytes,small", [(0, 1), (0, 0), (1, 0)])
+def test_chunked_levels_regression_bit_exact(gpu, level_bytes, small):
     """A level budget of 1 byte leaves room for one (tree, node) at a time:
-    every level below the root is processed node by node, each histogrammed
-    directly.  The trees are the same as with the whole-level path."""
-    print_case("estimator", "chunked levels regression, level_bytes", level_bytes)
+    every level of the chain below the root is processed node by node, each
+    histogrammed directly.  The trees are the same as with the whole-level path
+    and with one launch per level (small, which has no level buffers)."""
+    print_case("estimator", "chunked levels regression, level_bytes, small", level_bytes, small)
     X, y = c1_data(4000, 12)
     kw = dict(num_bins=16, max_depth=6, n_estimators=3, learning_rate=0.3, min_child_weight=10)
     m = WarpGBM(**kw)
     m._engine_level_bytes = level_bytes
-    m.fit(X, y)
+    m._engine_tuning = {8: small}
+    n = tile_launches(lambda: m.fit(X, y))
+    # none / one a level / one for each of a level's nodes
+    assert n == (0 if small else 3 * (63 if level_bytes else 6))
     codes = oracle_codes(m, X)
     ref = gbm.Forest(**kw).fit_codes(codes, y)
     for i, (a, b) in enumerate(zip(m.forest, ref.forest)):
@@ -595,8 +605,8 @@ def test_chunked_levels_regression_bit_exact(gpu, level_bytes):
 
 @pytest.mark.parametrize("N,F,B,depth,classes", [
     (41, 3, 5, 3, 0), (1023, 20, 32, 5, 0), (1025, 30, 127, 7, 0), (4097, 512, 10, 3, 0),
-    (4097, 513, 10, 3, 0), (8193, 33, 63, 7, 3), (16_384, 40, 2, 6, 0), (20_480, 40, 16, 4, 0), (20_481, 9, 16, 4, 0),
-    (12_289, 17, 9, 10, 0)])
+    (4097, 513, 10, 3, 0), (8193, 33, 63, 7, 3), (16_384, 40, 2, 6, 0), (20_480, 40, 16, 4, 0),
+    (20_481, 9, 16, 4, 0), (12_289, 17, 9, 10, 0)])
 def test_one_launch_levels_equal_level_chain(gpu, N, F, B, depth, classes):
     """One-era rounds of few rows (one launch per level) grow the level chain's
     trees: rows-per-thread remainders, the row and (feature, tree) limits, deep
@@ -694,7 +704,9 @@ def test_chunked_levels_multiclass_and_eras_bit_exact(gpu):
               learning_rate=0.3, min_child_weight=5)
     m = WarpGBM(**kw)
     m._engine_level_bytes = 40_000  # a few (tree, node)s per chunk
-    m.fit(X, labels)
+    m._engine_tuning = {8: 0}
+    # (two rounds of four levels, some of them in chunks)
+    assert tile_launches(lambda: m.fit(X, labels)) > 2 * 4
     codes = oracle_codes(m, X)
     ref = gbm.Forest(**kw).fit_codes(codes, labels)
     for i, (a, b) in enumerate(zip(m.forest, ref.forest)):

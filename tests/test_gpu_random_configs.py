@@ -9,8 +9,9 @@ colsample_bytree, min_child_weight, min_split_gain (0, small, large: the
 engine's `crit > min_split_gain` masks, and the DES rule that a node whose
 max-agreement candidates all fail it is a leaf), L2_reg (0, the default,
 1), float or pre-binned int8 input, and the objective (regression, or
-softmax with 3 classes).  Bar: identical tree dicts, bit-exact predictions
-and importances."""
+softmax with 3 classes).  One-era cases run twice, as the dispatch has them and
+in the level chain that larger data takes.  Bar: identical tree dicts, bit-exact
+predictions and importances."""
 import numpy as np
 import pytest
 
@@ -48,13 +49,15 @@ def draw_case(seed):
     return c, rng
 
 
-CASES = list(range(64))
+# one-era cases (small enough for one launch per level) also in the level chain
+CASES = [(seed, chain) for seed in range(64) for chain in (False, True)
+         if not chain or draw_case(seed)[0]["E"] == 1]
 
 
-@pytest.mark.parametrize("seed", CASES)
-def test_random_config_bit_exact(gpu, seed):
+@pytest.mark.parametrize("seed,chain", CASES)
+def test_random_config_bit_exact(gpu, seed, chain):
     c, rng = draw_case(seed)
-    print_case("random config", seed, c)
+    print_case("random config", seed, c, "level chain" if chain else "")
     N, F, B, E = c["N"], c["F"], c["B"], c["E"]
     if c["prebinned"]:
         X = rng.integers(0, B, (N, F)).astype(np.int8)
@@ -70,12 +73,16 @@ def test_random_config_bit_exact(gpu, seed):
               min_split_gain=c["msg"], L2_reg=c["l2"])
     if c["objective"] == "regression":
         y = (signal + 0.3 * rng.standard_normal(N)).astype(F32)
-        m = WarpGBM(random_state=seed, **kw).fit(X, y, era_id=era)
+        m = WarpGBM(random_state=seed, **kw)
+        m._engine_tuning = {8: 0} if chain else {}
+        m.fit(X, y, era_id=era)
         target = y
     else:
         labels = np.digitize(signal + 0.3 * rng.standard_normal(N),
                              np.quantile(signal, [1 / 3, 2 / 3])).astype(np.int64)
-        m = WarpGBM(objective="multiclass", random_state=seed, **kw).fit(X, labels)
+        m = WarpGBM(objective="multiclass", random_state=seed, **kw)
+        m._engine_tuning = {8: 0} if chain else {}
+        m.fit(X, labels)
         target = labels
     if c["prebinned"]:
         codes = X
