@@ -55,7 +55,7 @@ __device__ __forceinline__ uint32_t q_bucket(float x) {
   return b < kQBuckets - 1 ? b : kQBuckets - 1;
 }
 // byte address of a lane's entry for bucket b in a [256][64] word table (byte
-// b >> 8 of word (b & 255) * 64 + lane): one permute and one or
+// b >> 8 of word (b & 255) * 64 + lane): a byte permute and a bitwise or
 __device__ __forceinline__ uint32_t q_slot_addr(uint32_t b, uint32_t lane4) {
   return __builtin_amdgcn_perm(0u, b, 0x0c0c0001u) | lane4;
 }
