@@ -669,7 +669,9 @@ def test_one_launch_levels_where_they_pay(gpu, N, F, B, classes, small):
 
 @pytest.mark.parametrize("N,F,classes", [(20_481, 3, 0), (102_400, 3, 0), (102_401, 3, 0),
                                          (204_801, 3, 0), (204_802, 2, 0), (25_600, 1000, 0),
-                                         (34_134, 5, 3)])
+                                         (34_134, 5, 3), (131_072, 3, 0), (131_073, 3, 0),
+                                         (262_145, 3, 0), (262_146, 2, 0), (32_769, 1000, 0),
+                                         (43_691, 5, 3)])
 def test_level_tile_rows_bit_exact(gpu, N, F, classes):
     """Levels with tiles of 512 rows (few workgroups) grow the trees that tiles
     of 1024 grow, on both sides of the row limit for the root and the levels

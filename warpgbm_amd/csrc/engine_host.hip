@@ -518,15 +518,15 @@ static int ensure_tiles(Engine* e, int64_t max_tiles) {
 }
 
 // A whole level's tiles have 1024 rows at least (a tile's partial is up to
-// 64 KB, written and read again), 512 where those would give fewer than 100
-// of the 256 CUs a workgroup: the launch then takes as long as one tile's
-// rows, 15 us at 1024.  Us per round with 1024 / 512 / 256 rows: 100003 x 200,
-// 10 bins, depth 3 139 / 126 / 127; 100000 x 100, 32 bins, depth 6 253 / 241 /
-// 249; 50000 x 1000, depth 5 265 / 254 / 273; 40000 x 100, 3 classes 216 / 207
-// / 212; with more workgroups than that 512 rows lose: 50000 x 300, 127 bins
-// (122 workgroups below the root) 484 / 490 / 527; 500000 x 60, 10 bins 234 /
-// 246 / 284.  Era segments keep 1024 (50000 x 100, 3 eras 350 / 355 / 391).
-constexpr int64_t kHistIdleRows = 100 * 1024;
+// 64 KB, written and read again), 512 while those are at most one a CU: with
+// 1024 half of the CUs have no tile, and the launch takes as long as one tile's
+// rows, 15 us.  Us of a root level with tiles of 1024 / 512 rows, at workgroups of
+// 1024 rows: 200 x 10 bins 100 56 / 53, 124 57 / 55, 130 58 / 60; 1000 x 32 bins 100 63
+// / 60, 124 64 / 60, 130 64 / 64, 150 64 / 66; 60 x 32 bins 52 / 52, 54 / 54, 53 / 55;
+// 100 x 127 bins 90 / 91, 91 / 93, 91 / 94 (the levels below gain as much).  256
+// rows were no faster anywhere; era segments keep 1024 (50000 x 100, 3 eras 350 /
+// 355 / 391).
+constexpr int64_t kHistIdleRows = 128 * 1024;
 
 // histogram tiles of level d (the root, or the key pairs of every split: the
 // smaller child, or both children when one takes a finer shift): tile rows,
