@@ -297,8 +297,10 @@ int wgbm_engine_round(wgbm_engine* eng, const void* target, float* pred, const i
  * (node, era) segment's child ranges and leaves its sums for the node scan,
  * no block prefix, default; 0 = route, block prefix, node scan, scatter);
  * key 8 = one-era rounds of at most 20480 rows and 512 (feature, tree)s (1 =
- * one launch per level, default; 0 = the level chain; setting any of keys 1
- * to 7 takes the level chain too, whose parts they choose).
+ * one launch per level where that is the faster, default; 0 = the level chain;
+ * setting any of keys 1 to 7 takes the level chain too, whose parts they choose).
+ * Keys 1 and 2 size the era path's tile buffers again (a synchronisation and an
+ * allocation; without room the levels go without tiles).
  * Set before the first round; every setting grows the same trees. */
 int wgbm_engine_set_tuning(wgbm_engine* eng, int32_t key, int64_t value);
 void wgbm_engine_destroy(wgbm_engine* eng);
