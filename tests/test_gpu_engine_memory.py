@@ -63,10 +63,16 @@ def free_bytes():
 
 
 def fill_memory():
-    """All device memory but about 200 MB (what was freed before comes back late)."""
-    hog = []
-    while free_bytes() > 250_000_000:
-        hog.append(torch.empty(free_bytes() - 200_000_000, dtype=torch.uint8, device=dev))
+    """All device memory but about 300 MB (what was freed before comes back late,
+    and the largest piece that can be had may be less than what is free)."""
+    hog, most = [], 1 << 62
+    while (left := free_bytes() - 300_000_000) > 50_000_000:
+        try:
+            hog.append(torch.empty(min(left, most), dtype=torch.uint8, device=dev))
+        except torch.OutOfMemoryError:
+            most = min(left, most) // 2
+            if most < 50_000_000:
+                break
     return hog
 
 
